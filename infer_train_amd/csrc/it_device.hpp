@@ -91,6 +91,21 @@ __device__ __forceinline__ float group_max(float x) {
   return x;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave (DPP: row shifts within
+// each 16-lane row, then row broadcasts of lanes 15 and 31).  Lanes a DPP
+// source does not reach add 0 (bound_ctrl, or the disabled banks and rows,
+// which return the old operand 0).
+__device__ __forceinline__ int wave_inclusive_sum(int x) {
+  int v = x + __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);          // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, x, 0x113, 0xf, 0xf, true);          // row_shr:3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xe, false);         // row_shr:4, banks 1-3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xc, false);         // row_shr:8, banks 2-3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);         // row_bcast:15, rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);         // row_bcast:31, rows 2-3
+  return v;
+}
+
 // Load helpers: 16-byte vector loads/stores on raw byte addresses.
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ void st16(void* p, uint4 v) { *reinterpret_cast<uint4*>(p) = v; }

@@ -80,6 +80,7 @@ struct PrefillArgs {
   float scale_log2;
   int n_heads, n_kv_heads, group, q_tiles, max_blocks, log2_bs, causal, out_f32;
   int n_qb;               // query blocks per (sequence, KV head)
+  int n_seqs;
 };
 
 // Query tiles per workgroup for a GQA group: up to 8 waves of work.
@@ -129,13 +130,13 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 }
 // acc + lo + hi of a packed bf16 / f16 pair (v_dot2c_f32_*).
 template <bool kBf16>
-__device__ __forceinline__ float dot2_ones(uint32_t w, float acc) {
+__device__ __forceinline__ float dot2_ones(uint32_t w, float acc, uint32_t ones) {
   if constexpr (kBf16) {
     typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, w), __builtin_bit_cast(bf2, 0x3f803f80u), acc, false);
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, w), __builtin_bit_cast(bf2, ones), acc, false);
   } else {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, w), __builtin_bit_cast(h2, 0x3c003c00u), acc, false);
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, w), __builtin_bit_cast(h2, ones), acc, false);
   }
 }
 // max / sum of x over this lane and lane ^ 32 (v_permlane32_swap, no LDS).
@@ -148,6 +149,128 @@ __device__ __forceinline__ float sum_halves(float x) {
   return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
+// Units (sequence, KV head, query block) in longest-first order: by 64-key
+// blocks to read, most first; ties by sequence, query block, KV head.  The
+// lengths are on the device, so every wave finds its unit itself: lane i
+// holds sequences i, 64 + i, ...; count(L), the units of at least L blocks,
+// is a closed form per sequence and a wave sum; a binary search over L finds
+// the rank's block count, a prefix sum its sequence.  ~10 wave sums, 0.5 us,
+// against units of 2.2 us per key block.
+// Ids dealt pair by pair instead (all blocks of a sequence's KV heads on the
+// XCDs its number falls to) left the XCD holding the longest prompt working
+// alone: six prompts of 65 to 1500 tokens (28 heads over 4) 110 us.
+constexpr int kOrderSeqs = 256;
+constexpr int kFewSeqs = 24;
+struct PrefillUnit {
+  int b, kvh, qb;           // sequence, KV head, query block
+  int q_begin, q_len, ctx;  // of the sequence
+};
+__device__ __forceinline__ bool unit_of_rank(const PrefillArgs& a, int r, PrefillUnit& u) {
+  constexpr int kC = kOrderSeqs / 64;
+  const int lane = int(threadIdx.x & 63);
+  const int wg_q = kQB * a.q_tiles, sh = 31 - __builtin_clz(unsigned(wg_q));  // q_tiles: 1, 2, 4 or 8
+  const int hkv = a.n_kv_heads;
+  int first[kC], qlen[kC], before[kC], nq[kC];  // chunk's first row, rows, keys before it, query blocks
+  int top = 0, nq_all = 0;
+#pragma unroll
+  for (int c = 0; c < kC; ++c) {
+    const int s = 64 * c + lane;
+    first[c] = qlen[c] = before[c] = nq[c] = 0;
+    if (s < a.n_seqs) {
+      first[c] = a.cu_q[s];
+      qlen[c] = a.cu_q[s + 1] - first[c];
+      before[c] = a.ctx_lens[s] - qlen[c];
+      nq[c] = min(a.n_qb, (max(qlen[c], 0) + wg_q - 1) >> sh);
+    }
+    if (nq[c] > 0) top = max(top, before[c] + (a.causal ? min(qlen[c], nq[c] << sh) : qlen[c]));
+    nq_all += nq[c];
+  }
+  auto total = [](int x) { return __builtin_amdgcn_readlane(wave_inclusive_sum(x), 63); };
+  const int n_units = hkv * total(nq_all);
+  if (r >= n_units) return false;
+  // A batch of equal sequences (or one): later query blocks never read fewer
+  // keys, so the order is by query block (config 3: 1 us a workgroup less
+  // than the search below).
+  const int q0 = __builtin_amdgcn_readfirstlane(qlen[0]), b0 = __builtin_amdgcn_readfirstlane(before[0]);
+  bool differs = false;
+#pragma unroll
+  for (int c = 0; c < kC; ++c) differs |= 64 * c + lane < a.n_seqs && (qlen[c] != q0 || before[c] != b0);
+  if (__builtin_amdgcn_ballot_w64(differs) == 0) {
+    const int per = a.n_seqs * hkv, k = r / per, p = r - k * per;
+    u.qb = __builtin_amdgcn_readfirstlane(nq[0]) - 1 - k;
+    u.b = p / hkv, u.kvh = p - u.b * hkv;
+    u.q_begin = __builtin_amdgcn_readfirstlane(first[0]) + u.b * q0;
+    u.q_len = q0, u.ctx = b0 + q0;
+    return true;
+  }
+  // Query blocks of this lane's sequence c with at least L key blocks: those
+  // whose last row's key end, before + min(qlen, (qb + 1) wg_q), is past
+  // 64 (L - 1) (a chunk that attends everything: its whole context).
+  auto at_least = [&](int c, int L) {
+    if (L <= 0) return nq[c];
+    const int x = kKB * (L - 1) - before[c];
+    if (x >= qlen[c]) return 0;
+    return (x < 0 || !a.causal) ? nq[c] : max(nq[c] - (x >> sh), 0);
+  };
+  auto count = [&](int L) {
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kC; ++c)
+      if (64 * c < a.n_seqs) n += at_least(c, L);
+    return hkv * total(n);
+  };
+  // Past the most blocks any unit has (+ 2: the float of a count of 2^24 or more may be one less).
+  int lo = 0, hi = __builtin_amdgcn_readfirstlane(int(group_max<64>(float((max(top, 0) + kKB - 1) / kKB)))) + 2;
+  int past = 0;  // count(hi)
+  if (a.n_seqs <= kFewSeqs) {
+    // Few sequences: 64 values of L at a time, one per lane, the sequences
+    // one after another (config 3's 8: 0.3 us a workgroup less than below).
+    while (hi - lo > 1) {
+      const int step = (hi - lo + 63) >> 6;
+      const int L = lo + step * (lane + 1);
+      int n = 0;
+      for (int s = 0; s < a.n_seqs; ++s) {
+        const int ql = __builtin_amdgcn_readlane(qlen[0], s), nb = __builtin_amdgcn_readlane(nq[0], s);
+        const int x = kKB * (L - 1) - __builtin_amdgcn_readlane(before[0], s);
+        n += x >= ql ? 0 : (x < 0 || !a.causal) ? nb : max(nb - (x >> sh), 0);
+      }
+      n *= hkv;
+      const int k = int(__popcll(__builtin_amdgcn_ballot_w64(n > r && L < hi)));  // a prefix of the lanes
+      lo += step * k;
+      if (k < 64 && lo + step < hi) hi = lo + step, past = __builtin_amdgcn_readlane(n, k);
+    }
+  } else {
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1, n = count(mid);
+      if (n > r) lo = mid;
+      else hi = mid, past = n;
+    }
+  }
+  int base = past;
+#pragma unroll
+  for (int c = 0; c < kC; ++c) {
+    if (64 * c >= a.n_seqs) break;
+    const int longer = at_least(c, lo);
+    const int mine = hkv * (longer - at_least(c, hi));
+    const int incl = wave_inclusive_sum(mine);
+    const int all = __builtin_amdgcn_readlane(incl, 63);
+    if (r < base + all) {
+      const int idx = int(__popcll(__builtin_amdgcn_ballot_w64(base + incl <= r)));
+      const int k = r - base - __builtin_amdgcn_readlane(incl - mine, idx);
+      u.b = 64 * c + idx;
+      u.qb = k / hkv;
+      u.kvh = k - u.qb * hkv;
+      u.qb += __builtin_amdgcn_readlane(nq[c] - longer, idx);
+      u.q_begin = __builtin_amdgcn_readlane(first[c], idx);
+      u.q_len = __builtin_amdgcn_readlane(qlen[c], idx);
+      u.ctx = __builtin_amdgcn_readlane(before[c], idx) + u.q_len;
+      return true;
+    }
+    base += all;
+  }
+  return false;
+}
+
 // W: waves per workgroup (G query heads x QT query tiles).
 // kTab: the block-table row is copied into LDS after the rings (it fits).
 template <bool kBf16, int W, bool kTab>
@@ -155,31 +278,38 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // K ring, V ring, [table]
   constexpr int kDmaPerWave = (16 + W - 1) / W;  // 1 KiB loads per wave per plane (16 per plane)
   // Workgroup id -> (sequence, KV head, query block).  The dispatcher deals
-  // ids to the 8 XCDs round-robin; the ids are remapped so that all query
-  // blocks of one (sequence, KV head), which stream the same K/V pages, run
-  // on one XCD and share its L2 (in id order each XCD would fetch every
-  // sequence's pages).  In causal attention later query blocks see more
-  // keys, so each XCD takes its units longest first: the k-th workgroup of
-  // an XCD holding ppx whole (sequence, KV head) pairs takes query rank
-  // k / ppx of pair k % ppx.  Workgroups start in id order on whichever CU
-  // frees first, so a CU whose first workgroup was short takes the longest
-  // one left (config 3, two workgroups per CU: 166 against 174 us with
-  // query blocks in pair order).
-  const int n_full = int(gridDim.x) & ~7;
-  const int id = blockIdx.x;
-  const int per_xcd = n_full >> 3;
-  int k = id >> 3;
-  if (per_xcd > 0 && per_xcd % a.n_qb == 0) {
-    const int ppx = per_xcd / a.n_qb;
-    k = (k % ppx) * a.n_qb + k / ppx;
+  // ids to the 8 XCDs round-robin, and a CU takes its next workgroup when its
+  // first ends.  Up to kOrderSeqs sequences: id = rank in the longest-first
+  // order (unit_of_rank), so every XCD gets the same share of long and short
+  // units whatever the sequences' lengths.
+  PrefillUnit u;
+  if (a.n_seqs <= kOrderSeqs) {
+    if (!unit_of_rank(a, int(blockIdx.x), u)) return;  // uniform
+  } else {
+    // More sequences: ids are remapped so that all query blocks of one
+    // (sequence, KV head), which stream the same K/V pages, run on one XCD
+    // and share its L2; an XCD holding ppx whole pairs takes query rank
+    // k / ppx of pair k % ppx, its longest causal blocks first.
+    const int n_full = int(gridDim.x) & ~7;
+    const int id = blockIdx.x;
+    const int per_xcd = n_full >> 3;
+    int k = id >> 3;
+    if (per_xcd > 0 && per_xcd % a.n_qb == 0) {
+      const int ppx = per_xcd / a.n_qb;
+      k = (k % ppx) * a.n_qb + k / ppx;
+    }
+    const int unit = id < n_full ? (id & 7) * per_xcd + k : id;
+    const int pair = unit / a.n_qb;
+    u.qb = a.n_qb - 1 - (unit - pair * a.n_qb);
+    u.kvh = pair % a.n_kv_heads, u.b = pair / a.n_kv_heads;
+    u.q_begin = a.cu_q[u.b], u.q_len = a.cu_q[u.b + 1] - u.q_begin, u.ctx = a.ctx_lens[u.b];
   }
-  const int unit = id < n_full ? (id & 7) * per_xcd + k : id;
-  const int pair = unit / a.n_qb;
-  const int qb = a.n_qb - 1 - (unit - pair * a.n_qb);
-  const int kvh = pair % a.n_kv_heads, b = pair / a.n_kv_heads;
-  const int q_begin = a.cu_q[b];
-  const int q_len = a.cu_q[b + 1] - q_begin;
-  const int ctx = a.ctx_lens[b];
+  // Wave-uniform, and in scalar registers: left to the compiler (their last
+  // definitions sit in a loop) they took vector ones, and the main loop ran
+  // 7% slower.
+  auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  const int b = uni(u.b), kvh = uni(u.kvh), qb = uni(u.qb);
+  const int q_begin = uni(u.q_begin), q_len = uni(u.q_len), ctx = uni(u.ctx);
   const int wg_q = kQB * a.q_tiles;  // query positions per workgroup
   if (qb * wg_q >= q_len) return;    // uniform
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -382,6 +512,11 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   v16f s[2];     // S^T of the block the next softmax phase consumes
   uint4 pk[2][2];  // its probabilities, packed: [tile][k-step], 8 each
 
+  // A pair of 16-bit ones, in a register (as a literal it makes each v_dot2c
+  // an 8-byte instruction).
+  uint32_t ones = kBf16 ? 0x3f803f80u : 0x3c003c00u;
+  asm volatile("" : "+s"(ones));
+
   // Softmax phase of key block kb (VALU only): block max, lazy rescale of
   // o and l, probabilities into pk, their sum into l.  masked: keys past
   // lim_of(kb) are not visible (blocks below n_vis are whole).
@@ -422,7 +557,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
         for (int h = 0; h < 4; ++h) {
           w[h] = pack2<kBf16>(p[2 * h], p[2 * h + 1]);
           // The sum is taken over the rounded probabilities the MFMA uses.
-          bsum[h & 1] = dot2_ones<kBf16>(w[h], bsum[h & 1]);
+          bsum[h & 1] = dot2_ones<kBf16>(w[h], bsum[h & 1], ones);
         }
         pk[n][t] = make_uint4(w[0], w[1], w[2], w[3]);
       }
@@ -533,6 +668,11 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   uint4 tr[kTu][2];
   if (wave < 4) {
     softmax_phase(0, true, -INFINITY);
+    // The place of this loop's code is fixed: it ran 7% slower (one sequence of
+    // 16500 keys: 445 us against 417) in every build that had its first
+    // instruction 4 bytes off a multiple of 8, and any change before it moved
+    // it there.  (s_nop fills the gap, once per workgroup.)
+    asm volatile(".p2align 6");
 #pragma nounroll
     for (int kb = 0; kb < u_end; ++kb) {
       barrier_after_softmax(true);
@@ -554,6 +694,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
       transpose_store(kb + 1, tr);
     }
   } else {
+    asm volatile(".p2align 6");
 #pragma nounroll
     for (int kb = 0; kb < u_end; ++kb) {
       const float ninf = barrier_before_softmax(true);
@@ -680,6 +821,7 @@ extern "C" int32_t it_paged_prefill(const it_kv_cache* c, const void* q, int32_t
   a.out_f32 = out_dtype == IT_F32;
   const int wg_q = kQB * a.q_tiles;
   a.n_qb = (max_q_len + wg_q - 1) / wg_q;
+  a.n_seqs = n_seqs;
   const int64_t n_wg = int64_t(a.n_qb) * c->n_kv_heads * n_seqs;
   if (n_wg > INT32_MAX) return fail(IT_INVALID_INPUT, "%s: %lld workgroups (max 2^31 - 1)", who, (long long)n_wg);
   const dim3 grid(static_cast<unsigned>(n_wg), 1u, 1u);

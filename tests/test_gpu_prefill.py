@@ -187,3 +187,22 @@ def test_prefill_config3_rows():
         up = hi[:, pos, :].transpose(1, 0, 2)[:, :, None, :]
         dn = lo[:, pos, :].transpose(1, 0, 2)[:, :, None, :]
         assert np.all(o <= up + 1e-4) and np.all(o >= dn - 1e-4), f"config3 seq {s}: outside the V hull"
+
+
+@pytest.mark.parametrize("n_seqs,hq,hkv,causal", [(2, 7, 1, True), (63, 8, 1, True), (64, 4, 2, False), (65, 8, 1, True),
+                                                  (256, 8, 1, True), (257, 8, 1, True)])
+def test_prefill_unit_order_ragged(n_seqs, hq, hkv, causal):
+    """Workgroups find their unit in the longest-first order over 64-sequence
+    chunks (up to 256 sequences; more take ids in pair order): batches at the
+    chunks' edges, with empty chunks, chunk lengths of one row, whole prompts
+    and long cached prefixes.  Every row against the oracle, so every unit is
+    computed, and by nobody else (a unit missed leaves its rows unwritten)."""
+    rng = np.random.RandomState(n_seqs)
+    q_lens = rng.choice([0, 1, 31, 32, 33, 65, 100], n_seqs)
+    q_lens[0] = 97
+    ctx = q_lens + rng.choice([0, 1, 63, 64, 200], n_seqs)
+    ctx[0] += 300
+    dev, ref, tables, ctx, cu, q, td = _setup(orc.BF16, hq, hkv, ctx, q_lens, seed=500 + n_seqs)
+    out, scale = _run(dev, tables, ctx, cu, q, td, hq, causal=causal)
+    want = ref.prefill(widen(q, orc.BF16), hq, cu, tables, ctx, scale, causal=causal)
+    assert_close(from_dev(out), want, RTOL, ATOL, what=f"prefill order n_seqs={n_seqs}")
