@@ -425,6 +425,22 @@ int32_t it_paged_prefill(const it_kv_cache* cache, const void* q, int32_t q_dtyp
                          const int32_t* cu_q, int32_t max_q_len, const int32_t* block_tables,
                          int32_t max_blocks, const int32_t* ctx_lens, int32_t n_seqs, float scale,
                          int32_t causal, void* out, int32_t out_dtype, void* stream);
+/* Bytes of device workspace with which it_paged_prefill_ws can cut a call's
+ * work over the keys; 0 if it would not (a launch of this size fills the
+ * device without).  Bounded: at most 70 MB. */
+size_t it_paged_prefill_workspace(int32_t n_heads, int32_t n_kv_heads, int32_t n_seqs, int32_t max_q_len,
+                                  int32_t max_blocks, int32_t block_size);
+/* it_paged_prefill with a workspace (device, 256-byte aligned,
+ * it_paged_prefill_workspace(...) bytes; NULL = none).  When the sequences'
+ * lengths leave the device with few workgroups (a chunk of one long
+ * context), the keys of each query block are divided among several, whose
+ * fp32 partial (m, l, O) go through the workspace to a second kernel that
+ * merges them. */
+int32_t it_paged_prefill_ws(const it_kv_cache* cache, const void* q, int32_t q_dtype, int32_t n_heads,
+                            const int32_t* cu_q, int32_t max_q_len, const int32_t* block_tables,
+                            int32_t max_blocks, const int32_t* ctx_lens, int32_t n_seqs, float scale,
+                            int32_t causal, void* ws, size_t ws_bytes, void* out, int32_t out_dtype,
+                            void* stream);
 
 /* CoreOperator::FlashAttention as ArmCpuBackend executes it
  * (src/backend/arm.rs:304-370): every one of n_heads query heads attends

@@ -27,8 +27,9 @@
 // VALU work at the same time.  Fully visible blocks (every key precedes
 // every query of the workgroup and kend) run a loop without per-key masks;
 // the blocks the causal diagonal or kend cut run a masked copy of it.
-// Workgroups are placed so that the query blocks of one (sequence, KV head)
-// share an XCD and its L2.
+// Workgroups take their units longest first over all sequences; where that
+// leaves CUs idle and the caller gave a workspace, a unit's keys are cut into
+// several workgroups, whose partials paged_prefill_combine merges.
 // K and V blocks (16 KiB each) are staged in LDS by direct global->LDS loads
 // into rings of 3 K and 3 V slots, issued three blocks ahead; 16-byte chunks
 // are XOR-swizzled by row so MFMA operand reads are conflict-free.  Each V
@@ -38,6 +39,9 @@
 // the vector-memory counter that orders the rings).  Online softmax in fp32
 // (exp2 domain), accumulators fp32.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <climits>
 
 #include "it_device.hpp"
 #include "it_internal.hpp"
@@ -52,6 +56,7 @@ constexpr int kRowB = kD * 2;         // bytes per K/V row
 constexpr int kPlaneB = kKB * kRowB;  // 16 KiB
 constexpr int kRingK = 3;             // K slots
 constexpr int kRingV = 3;             // V slots (row-major, as loaded)
+static_assert(kRingK == kRingV, "one slot index serves both rings");
 // V^T slots: row d holds dim d of the block's 64 keys, key k at position
 // vt_pos(k); rows padded to 144 bytes so both the 16-byte operand reads (8
 // consecutive rows per pass) and the 4-byte transpose stores are
@@ -81,6 +86,9 @@ struct PrefillArgs {
   int n_heads, n_kv_heads, group, q_tiles, max_blocks, log2_bs, causal, out_f32;
   int n_qb;               // query blocks per (sequence, KV head)
   int n_seqs;
+  int max_tiles;          // tiles the workspace holds; 0: units are not split
+  float4* ws_o;           // [max_tiles][waves][16][64]: a wave's O^T registers, 16 bytes of each lane
+  float2* ws_ml;          // [max_tiles][waves][64]: (max, sum) of each lane's query
 };
 
 // Query tiles per workgroup for a GQA group: up to 8 waves of work.
@@ -152,88 +160,120 @@ __device__ __forceinline__ float sum_halves(float x) {
 // Units (sequence, KV head, query block) in longest-first order: by 64-key
 // blocks to read, most first; ties by sequence, query block, KV head.  The
 // lengths are on the device, so every wave finds its unit itself: lane i
-// holds sequences i, 64 + i, ...; count(L), the units of at least L blocks,
-// is a closed form per sequence and a wave sum; a binary search over L finds
-// the rank's block count, a prefix sum its sequence.  ~10 wave sums, 0.5 us,
-// against units of 2.2 us per key block.
+// holds sequence i; count(L), the units of at least L blocks, is a closed
+// form per sequence and a sum over the lanes; a search over L finds the
+// rank's block count, a prefix sum its sequence: 0.5-1 us, against units of
+// 1.7-2.2 us per key block.
 // Ids dealt pair by pair instead (all blocks of a sequence's KV heads on the
 // XCDs its number falls to) left the XCD holding the longest prompt working
-// alone: six prompts of 65 to 1500 tokens (28 heads over 4) 110 us.
-constexpr int kOrderSeqs = 256;
+// alone: six prompts of 65 to 1500 tokens (28 heads over 4) 110 us, 72 so.
+// Batches of more sequences than a wave has lanes keep that older order.
+constexpr int kOrderSeqs = 64;
 constexpr int kFewSeqs = 24;
 struct PrefillUnit {
   int b, kvh, qb;           // sequence, KV head, query block
   int q_begin, q_len, ctx;  // of the sequence
 };
-__device__ __forceinline__ bool unit_of_rank(const PrefillArgs& a, int r, PrefillUnit& u) {
-  constexpr int kC = kOrderSeqs / 64;
-  const int lane = int(threadIdx.x & 63);
-  const int wg_q = kQB * a.q_tiles, sh = 31 - __builtin_clz(unsigned(wg_q));  // q_tiles: 1, 2, 4 or 8
-  const int hkv = a.n_kv_heads;
-  int first[kC], qlen[kC], before[kC], nq[kC];  // chunk's first row, rows, keys before it, query blocks
-  int top = 0, nq_all = 0;
-#pragma unroll
-  for (int c = 0; c < kC; ++c) {
-    const int s = 64 * c + lane;
-    first[c] = qlen[c] = before[c] = nq[c] = 0;
-    if (s < a.n_seqs) {
-      first[c] = a.cu_q[s];
-      qlen[c] = a.cu_q[s + 1] - first[c];
-      before[c] = a.ctx_lens[s] - qlen[c];
-      nq[c] = min(a.n_qb, (max(qlen[c], 0) + wg_q - 1) >> sh);
-    }
-    if (nq[c] > 0) top = max(top, before[c] + (a.causal ? min(qlen[c], nq[c] << sh) : qlen[c]));
-    nq_all += nq[c];
+struct UnitOrder {
+  int first, qlen, before, nq;  // lane i's sequence: the chunk's first row, its rows, the keys before it, query blocks
+  int n_units;
+  int splits;  // workgroups a unit may be cut over its keys for (1: none is)
+};
+// Key cuts.  A launch of few units (one sequence's chunk: 500 rows of 32
+// heads over 8 are 64) leaves CUs idle while each unit streams its whole
+// context; cut over their keys into `splits` workgroups, whose partial (m, l,
+// O) the combine kernel merges, they fill the chip.  A cut costs its ring's
+// start, 132 KiB of partials written and read: about kCutCost key blocks of
+// time.  The cut count minimises rounds of workgroups x blocks of each, over
+// the units' mean and their longest; a unit keeps at least kCutMin blocks a
+// cut.  500 rows over 16500 keys: 4 cuts, 417 -> 156 us.
+constexpr int kCus = 256;
+constexpr int kMaxTiles = 512;
+constexpr int kMaxCuts = 16;
+constexpr int kCutCost = 5;
+constexpr int kCutMin = 8;
+__device__ __forceinline__ int key_blocks(int keys) { return max((keys + kKB - 1) >> 6, 0); }
+__device__ __forceinline__ int unit_cuts(int splits, int nkb) { return max(min(splits, nkb / kCutMin), 1); }
+
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_inclusive_sum(x), 63); }
+__device__ __forceinline__ int query_shift(const PrefillArgs& a) {  // log2 of a workgroup's query positions
+  return 5 + __builtin_ctz(unsigned(a.q_tiles));                    // q_tiles: 1, 2, 4 or 8
+}
+// Key end of the first / last query block of this lane's sequence.
+__device__ __forceinline__ int last_end(const PrefillArgs& a, const UnitOrder& o) {
+  return o.before + (a.causal ? min(o.qlen, o.nq << query_shift(a)) : o.qlen);
+}
+__device__ __forceinline__ int first_end(const PrefillArgs& a, const UnitOrder& o) {
+  return o.before + (a.causal ? min(o.qlen, 1 << query_shift(a)) : o.qlen);
+}
+// Most key blocks of a unit (+ 1: the float of 2^24 or more may be one less).
+__device__ __forceinline__ int most_blocks(const PrefillArgs& a, const UnitOrder& o) {
+  const int top = o.nq > 0 ? key_blocks(last_end(a, o)) : 0;
+  return __builtin_amdgcn_readfirstlane(int(group_max<64>(float(top)))) + 1;
+}
+
+__device__ __forceinline__ void load_order(const PrefillArgs& a, UnitOrder& o) {
+  const int lane = int(threadIdx.x & 63), sh = query_shift(a);
+  const int s = min(lane, a.n_seqs - 1);
+  o.first = a.cu_q[s];
+  o.qlen = a.cu_q[s + 1] - o.first;
+  o.before = a.ctx_lens[s] - o.qlen;
+  o.nq = lane < a.n_seqs ? min(a.n_qb, (max(o.qlen, 0) + (1 << sh) - 1) >> sh) : 0;
+  o.n_units = a.n_kv_heads * wave_total(o.nq);
+  o.splits = 1;
+  if (a.max_tiles > 0 && o.n_units > 0 && 2 * o.n_units <= a.max_tiles) {  // uniform
+    // Lane i prices i + 1 cuts, in 16ths of a key block's time.
+    const int most = most_blocks(a, o) - 1;
+    const int work = (o.nq * (key_blocks(first_end(a, o)) + key_blocks(last_end(a, o)))) >> 1;
+    const int S = lane + 1;
+    const int mean16 = int(int64_t(a.n_kv_heads) * wave_total(work) * 16 / o.n_units);
+    const int cut16 = S > 1 ? 16 * kCutCost : 0;
+    const int rounds = (o.n_units * S + kCus - 1) / kCus;
+    int cost = max(rounds * (mean16 / S + cut16), 16 * most / S + cut16);
+    if (S > kMaxCuts || (S > 1 && (o.n_units * S > a.max_tiles || most < kCutMin * S))) cost = INT_MAX;
+    // Only for a gain of a tenth.
+    if (S == 1) cost -= cost / 10;
+    const float c = -float(cost);
+    const float best = group_max<64>(c);
+    o.splits = __builtin_amdgcn_readfirstlane(int(__builtin_ctzll(__builtin_amdgcn_ballot_w64(c == best)))) + 1;
   }
-  auto total = [](int x) { return __builtin_amdgcn_readlane(wave_inclusive_sum(x), 63); };
-  const int n_units = hkv * total(nq_all);
-  if (r >= n_units) return false;
+}
+
+// The unit of rank r < o.n_units.
+__device__ __forceinline__ void unit_of_rank(const PrefillArgs& a, const UnitOrder& o, int r, PrefillUnit& u) {
+  const int lane = int(threadIdx.x & 63), sh = query_shift(a), hkv = a.n_kv_heads;
   // A batch of equal sequences (or one): later query blocks never read fewer
-  // keys, so the order is by query block (config 3: 1 us a workgroup less
-  // than the search below).
-  const int q0 = __builtin_amdgcn_readfirstlane(qlen[0]), b0 = __builtin_amdgcn_readfirstlane(before[0]);
-  bool differs = false;
-#pragma unroll
-  for (int c = 0; c < kC; ++c) differs |= 64 * c + lane < a.n_seqs && (qlen[c] != q0 || before[c] != b0);
-  if (__builtin_amdgcn_ballot_w64(differs) == 0) {
+  // keys, so the order is by query block (8 sequences: 1 us a workgroup less
+  // than the search below).  Lanes past the last sequence repeat it.
+  const int q0 = __builtin_amdgcn_readfirstlane(o.qlen), b0 = __builtin_amdgcn_readfirstlane(o.before);
+  if (__builtin_amdgcn_ballot_w64(o.qlen != q0 || o.before != b0) == 0) {
     const int per = a.n_seqs * hkv, k = r / per, p = r - k * per;
-    u.qb = __builtin_amdgcn_readfirstlane(nq[0]) - 1 - k;
+    u.qb = __builtin_amdgcn_readfirstlane(o.nq) - 1 - k;
     u.b = p / hkv, u.kvh = p - u.b * hkv;
-    u.q_begin = __builtin_amdgcn_readfirstlane(first[0]) + u.b * q0;
+    u.q_begin = __builtin_amdgcn_readfirstlane(o.first) + u.b * q0;
     u.q_len = q0, u.ctx = b0 + q0;
-    return true;
+    return;
   }
-  // Query blocks of this lane's sequence c with at least L key blocks: those
-  // whose last row's key end, before + min(qlen, (qb + 1) wg_q), is past
-  // 64 (L - 1) (a chunk that attends everything: its whole context).
-  auto at_least = [&](int c, int L) {
-    if (L <= 0) return nq[c];
-    const int x = kKB * (L - 1) - before[c];
-    if (x >= qlen[c]) return 0;
-    return (x < 0 || !a.causal) ? nq[c] : max(nq[c] - (x >> sh), 0);
+  // Query blocks of a sequence with at least L key blocks: those whose last
+  // row's key end, before + min(qlen, (qb + 1) wg_q), is past 64 (L - 1) (a
+  // chunk that attends everything: its whole context).
+  auto at_least = [&](int qlen, int before, int nq, int L) {
+    if (L <= 0) return nq;
+    const int x = kKB * (L - 1) - before;
+    return x >= qlen ? 0 : (x < 0 || !a.causal) ? nq : max(nq - (x >> sh), 0);
   };
-  auto count = [&](int L) {
-    int n = 0;
-#pragma unroll
-    for (int c = 0; c < kC; ++c)
-      if (64 * c < a.n_seqs) n += at_least(c, L);
-    return hkv * total(n);
-  };
-  // Past the most blocks any unit has (+ 2: the float of a count of 2^24 or more may be one less).
-  int lo = 0, hi = __builtin_amdgcn_readfirstlane(int(group_max<64>(float((max(top, 0) + kKB - 1) / kKB)))) + 2;
+  int lo = 0, hi = most_blocks(a, o) + 1;
   int past = 0;  // count(hi)
   if (a.n_seqs <= kFewSeqs) {
     // Few sequences: 64 values of L at a time, one per lane, the sequences
-    // one after another (config 3's 8: 0.3 us a workgroup less than below).
+    // one after another (8 sequences: 0.3 us a workgroup less than below).
     while (hi - lo > 1) {
       const int step = (hi - lo + 63) >> 6;
       const int L = lo + step * (lane + 1);
       int n = 0;
-      for (int s = 0; s < a.n_seqs; ++s) {
-        const int ql = __builtin_amdgcn_readlane(qlen[0], s), nb = __builtin_amdgcn_readlane(nq[0], s);
-        const int x = kKB * (L - 1) - __builtin_amdgcn_readlane(before[0], s);
-        n += x >= ql ? 0 : (x < 0 || !a.causal) ? nb : max(nb - (x >> sh), 0);
-      }
+      for (int s = 0; s < a.n_seqs; ++s)
+        n += at_least(__builtin_amdgcn_readlane(o.qlen, s), __builtin_amdgcn_readlane(o.before, s),
+                      __builtin_amdgcn_readlane(o.nq, s), L);
       n *= hkv;
       const int k = int(__popcll(__builtin_amdgcn_ballot_w64(n > r && L < hi)));  // a prefix of the lanes
       lo += step * k;
@@ -241,34 +281,45 @@ __device__ __forceinline__ bool unit_of_rank(const PrefillArgs& a, int r, Prefil
     }
   } else {
     while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1, n = count(mid);
+      const int mid = (lo + hi) >> 1, n = hkv * wave_total(at_least(o.qlen, o.before, o.nq, mid));
       if (n > r) lo = mid;
       else hi = mid, past = n;
     }
   }
-  int base = past;
+  const int longer = at_least(o.qlen, o.before, o.nq, lo);
+  const int mine = hkv * (longer - at_least(o.qlen, o.before, o.nq, hi));
+  const int incl = wave_inclusive_sum(mine);
+  // Inclusive prefixes do not decrease: the lanes at or below the rank are a
+  // prefix of the wave, the rank's sequence the next lane.
+  const int idx = min(int(__popcll(__builtin_amdgcn_ballot_w64(past + incl <= r))), a.n_seqs - 1);
+  const int k = r - past - __builtin_amdgcn_readlane(incl - mine, idx);
+  u.b = idx;
+  u.qb = k / hkv;
+  u.kvh = k - u.qb * hkv;
+  u.qb += __builtin_amdgcn_readlane(o.nq - longer, idx);
+  u.q_begin = __builtin_amdgcn_readlane(o.first, idx);
+  u.q_len = __builtin_amdgcn_readlane(o.qlen, idx);
+  u.ctx = __builtin_amdgcn_readlane(o.before, idx) + u.q_len;
+}
+
+// Keys the unit's query block needs: up to its last valid query's position.
+__device__ __forceinline__ int unit_keys(const PrefillArgs& a, int q_len, int ctx, int qb) {
+  const int wg_q = kQB * a.q_tiles;
+  return a.causal ? ctx - q_len + min(q_len, (qb + 1) * wg_q) : ctx;
+}
+
+// Normalise and store four dims of one query: O / l, zeros where no key was
+// seen (flash_attn.rs:66-71).
+template <bool kBf16>
+__device__ __forceinline__ void store4(const PrefillArgs& a, int64_t at, const float (&o)[4], float l, float inv) {
+  float v[4];
 #pragma unroll
-  for (int c = 0; c < kC; ++c) {
-    if (64 * c >= a.n_seqs) break;
-    const int longer = at_least(c, lo);
-    const int mine = hkv * (longer - at_least(c, hi));
-    const int incl = wave_inclusive_sum(mine);
-    const int all = __builtin_amdgcn_readlane(incl, 63);
-    if (r < base + all) {
-      const int idx = int(__popcll(__builtin_amdgcn_ballot_w64(base + incl <= r)));
-      const int k = r - base - __builtin_amdgcn_readlane(incl - mine, idx);
-      u.b = 64 * c + idx;
-      u.qb = k / hkv;
-      u.kvh = k - u.qb * hkv;
-      u.qb += __builtin_amdgcn_readlane(nq[c] - longer, idx);
-      u.q_begin = __builtin_amdgcn_readlane(first[c], idx);
-      u.q_len = __builtin_amdgcn_readlane(qlen[c], idx);
-      u.ctx = __builtin_amdgcn_readlane(before[c], idx) + u.q_len;
-      return true;
-    }
-    base += all;
+  for (int j = 0; j < 4; ++j) v[j] = l > 0.0f ? o[j] * inv : 0.0f;
+  if (a.out_f32) {
+    *reinterpret_cast<float4*>(static_cast<float*>(a.out) + at) = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + at) = make_uint2(pack2<kBf16>(v[0], v[1]), pack2<kBf16>(v[2], v[3]));
   }
-  return false;
 }
 
 // W: waves per workgroup (G query heads x QT query tiles).
@@ -283,8 +334,18 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   // order (unit_of_rank), so every XCD gets the same share of long and short
   // units whatever the sequences' lengths.
   PrefillUnit u;
+  int cut = 0, splits = 1;  // this workgroup's share of its unit's key blocks: cut of min(splits, ...)
   if (a.n_seqs <= kOrderSeqs) {
-    if (!unit_of_rank(a, int(blockIdx.x), u)) return;  // uniform
+    UnitOrder o;
+    load_order(a, o);
+    splits = o.splits;
+    int r = int(blockIdx.x);
+    if (splits > 1) {  // uniform
+      r /= splits;
+      cut = int(blockIdx.x) - r * splits;
+    }
+    if (r >= o.n_units) return;  // uniform
+    unit_of_rank(a, o, r, u);
   } else {
     // More sequences: ids are remapped so that all query blocks of one
     // (sequence, KV head), which stream the same K/V pages, run on one XCD
@@ -320,10 +381,14 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   const int qi = qb * wg_q + tile * kQB + col;
   const bool q_ok = qi < q_len;
   const int q_pos = ctx - q_len + qi;  // absolute position of this lane's query
-  // Keys this workgroup needs: up to its last valid query's position.
-  const int last_q = min(q_len, (qb + 1) * wg_q) - 1;
-  const int kend = a.causal ? min(ctx, ctx - q_len + last_q + 1) : ctx;
-  const int nkb = (kend + kKB - 1) / kKB;
+  // Keys this workgroup needs: its cut [kb0, nkb) of the unit's key blocks
+  // (the whole of them unless the unit is cut).
+  const int unit_end = unit_keys(a, q_len, ctx, qb);
+  const int unit_kb = key_blocks(unit_end);
+  const int cuts = unit_cuts(splits, unit_kb);
+  if (cut >= cuts) return;  // uniform
+  const int kb0 = unit_kb * cut / cuts, nkb = unit_kb * (cut + 1) / cuts;
+  const int kend = min(unit_end, nkb * kKB);
   const int first_pos = ctx - q_len + qb * wg_q;  // position of the workgroup's first query
   const int vis_end = a.causal ? min(kend, first_pos + 1) : kend;
   const int n_vis = max(vis_end, 0) / kKB;  // blocks every query of the workgroup sees whole
@@ -596,27 +661,29 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   // Prologue: (K(0), V(0)), (K(1), V(1)), (K(2), V(2)); V(0) transposed;
   // S^T of block 0.  A workgroup with no keys (nkb uniform) skips straight
   // to the zero output.
-  if (nkb > 0) {
+  if (nkb > kb0) {
   {
     int b0[kDmaPerWave], b1[kDmaPerWave];
-    page_ids(0, b0);
-    page_ids(1, b1);
-    page_ids(2, kblk);
-    dma_plane(k_head, 0, k_m0, b0);
-    dma_plane(v_head, 0, v_m0, b0);
-    dma_plane(k_head, 1, k_m0 + uint32_t(kPlaneB), b1);
-    dma_plane(v_head, 1, v_m0 + uint32_t(kPlaneB), b1);
-    dma_plane(k_head, 2, k_m0 + uint32_t(2 * kPlaneB), kblk);
-    dma_plane(v_head, 2, v_m0 + uint32_t(2 * kPlaneB), kblk);
-    page_ids(3, kblk);
+    page_ids(kb0, b0);
+    page_ids(kb0 + 1, b1);
+    page_ids(kb0 + 2, kblk);
+    const uint32_t s0 = uint32_t(kb0 % kRingK) * kPlaneB, s1 = uint32_t((kb0 + 1) % kRingK) * kPlaneB,
+                   s2 = uint32_t((kb0 + 2) % kRingK) * kPlaneB;
+    dma_plane(k_head, kb0, k_m0 + s0, b0);
+    dma_plane(v_head, kb0, v_m0 + s0, b0);
+    dma_plane(k_head, kb0 + 1, k_m0 + s1, b1);
+    dma_plane(v_head, kb0 + 1, v_m0 + s1, b1);
+    dma_plane(k_head, kb0 + 2, k_m0 + s2, kblk);
+    dma_plane(v_head, kb0 + 2, v_m0 + s2, kblk);
+    page_ids(kb0 + 3, kblk);
   }
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"n"(4 * kDmaPerWave) : "memory");
   {
     uint4 r[kTu][2];
-    transpose_read(0, r);
-    transpose_store(0, r);
+    transpose_read(kb0, r);
+    transpose_store(kb0, r);
   }
-  qk(0, s);
+  qk(kb0, s);
   // Ping-pong: waves 0-3 (one per SIMD) run step kb as the matrix phase of
   // block kb, a workgroup barrier, then the softmax phase of block kb + 1;
   // waves 4-7 run the softmax phase of block kb, the barrier, then the
@@ -664,17 +731,17 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   // (kb + 1) & 1 was last read by the matrix phases of step kb - 1.  (The
   // last step transposes the refilled copy of the last block; no step reads
   // it.)
-  const int u_end = max(n_vis - 1, 0);
+  const int u_end = max(n_vis - 1, kb0);
   uint4 tr[kTu][2];
   if (wave < 4) {
-    softmax_phase(0, true, -INFINITY);
+    softmax_phase(kb0, true, -INFINITY);
     // The place of this loop's code is fixed: it ran 7% slower (one sequence of
     // 16500 keys: 445 us against 417) in every build that had its first
     // instruction 4 bytes off a multiple of 8, and any change before it moved
     // it there.  (s_nop fills the gap, once per workgroup.)
     asm volatile(".p2align 6");
 #pragma nounroll
-    for (int kb = 0; kb < u_end; ++kb) {
+    for (int kb = kb0; kb < u_end; ++kb) {
       barrier_after_softmax(true);
       issue_step(kb);
       matrix_phase(kb);
@@ -696,7 +763,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   } else {
     asm volatile(".p2align 6");
 #pragma nounroll
-    for (int kb = 0; kb < u_end; ++kb) {
+    for (int kb = kb0; kb < u_end; ++kb) {
       const float ninf = barrier_before_softmax(true);
       issue_step(kb);
       transpose_read(kb + 1, tr);
@@ -724,24 +791,72 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   // ---- normalise and store ------------------------------------------------
   // o[dt][r] is dim 32 dt + 8 (r / 4) + 4 half + r % 4 of query col.
   const float l_tot = sum_halves(l_run);
+  if (cuts > 1) {  // uniform: this cut's partial, as it sits in the registers
+    float4* const wo = a.ws_o + (int64_t(blockIdx.x) * W + wave) * 16 * 64 + lane;
+#pragma unroll
+    for (int dt = 0; dt < kD / 32; ++dt)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        wo[(4 * dt + g4) * 64] = make_float4(o[dt][4 * g4], o[dt][4 * g4 + 1], o[dt][4 * g4 + 2], o[dt][4 * g4 + 3]);
+    a.ws_ml[(int64_t(blockIdx.x) * W + wave) * 64 + lane] = make_float2(m_run, l_tot);
+    return;
+  }
   if (!q_ok) return;
-  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;  // flash_attn.rs:66-71
+  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
   const int64_t orow = ((int64_t(q_begin) + qi) * a.n_heads + head) * kD;
 #pragma unroll
   for (int dt = 0; dt < kD / 32; ++dt)
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
-      const int dim = 32 * dt + 8 * g4 + 4 * half;
-      float v[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = l_tot > 0.0f ? o[dt][4 * g4 + j] * inv : 0.0f;
-      if (a.out_f32) {
-        *reinterpret_cast<float4*>(static_cast<float*>(a.out) + orow + dim) = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + orow + dim) =
-            make_uint2(pack2<kBf16>(v[0], v[1]), pack2<kBf16>(v[2], v[3]));
-      }
+      const float v[4] = {o[dt][4 * g4], o[dt][4 * g4 + 1], o[dt][4 * g4 + 2], o[dt][4 * g4 + 3]};
+      store4<kBf16>(a, orow + 32 * dt + 8 * g4 + 4 * half, v, l_tot, inv);
     }
+}
+
+// Merge the cuts of a unit: M = max m_c, O = sum O_c 2^(m_c - M) / sum l_c
+// 2^(m_c - M) (the rescaling of flash_attn.rs:42-71 across cuts).  grid.x =
+// rank of the unit, grid.y = wave of its workgroup; wave dt of this one
+// takes dims 32 dt .. 32 dt + 31.  Units that are not cut were stored by the
+// main kernel.
+template <bool kBf16>
+__global__ __launch_bounds__(64 * (kD / 32)) void paged_prefill_combine(PrefillArgs a, int n_waves) {
+  UnitOrder ord;
+  load_order(a, ord);
+  const int r = int(blockIdx.x), wave = int(blockIdx.y);
+  if (ord.splits == 1 || r >= ord.n_units) return;  // uniform
+  PrefillUnit u;
+  unit_of_rank(a, ord, r, u);
+  const int cuts = unit_cuts(ord.splits, key_blocks(unit_keys(a, u.q_len, u.ctx, u.qb)));
+  if (cuts == 1) return;  // uniform
+  const int lane = int(threadIdx.x & 63), dt = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int tile = wave / a.group, head = u.kvh * a.group + (wave - tile * a.group);
+  const int qi = (u.qb * a.q_tiles + tile) * kQB + (lane & 31);
+  const int64_t t0 = int64_t(r) * ord.splits * n_waves + wave;  // cut c: t0 + c n_waves
+  const float2* const ml = a.ws_ml + t0 * 64 + lane;
+  const float4* const wo = a.ws_o + (t0 * 16 + 4 * dt) * 64 + lane;
+  float M = -INFINITY;
+#pragma unroll 4
+  for (int c = 0; c < cuts; ++c) M = fmaxf(M, ml[int64_t(c) * n_waves * 64].x);
+  float acc[4][4] = {}, l = 0.0f;
+#pragma unroll 4
+  for (int c = 0; c < cuts; ++c) {
+    const float2 x = ml[int64_t(c) * n_waves * 64];
+    const float w = x.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(x.x - M);
+    l = fmaf(x.y, w, l);
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const float4 v = wo[(int64_t(c) * n_waves * 16 + g4) * 64];
+      acc[g4][0] = fmaf(v.x, w, acc[g4][0]);
+      acc[g4][1] = fmaf(v.y, w, acc[g4][1]);
+      acc[g4][2] = fmaf(v.z, w, acc[g4][2]);
+      acc[g4][3] = fmaf(v.w, w, acc[g4][3]);
+    }
+  }
+  if (qi >= u.q_len) return;
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const int64_t orow = ((int64_t(u.q_begin) + qi) * a.n_heads + head) * kD;
+#pragma unroll
+  for (int g4 = 0; g4 < 4; ++g4) store4<kBf16>(a, orow + 32 * dt + 8 * g4 + 4 * (lane >> 5), acc[g4], l, inv);
 }
 
 template <bool kBf16, int W, bool kTab>
@@ -764,20 +879,58 @@ hipError_t launch_prefill_w(const PrefillArgs& a, dim3 grid, hipStream_t s) {
 
 template <bool kBf16>
 hipError_t launch_prefill(const PrefillArgs& a, dim3 grid, hipStream_t s) {
-  switch (a.group * a.q_tiles) {
-    case 5: return launch_prefill_w<kBf16, 5>(a, grid, s);
-    case 6: return launch_prefill_w<kBf16, 6>(a, grid, s);
-    case 7: return launch_prefill_w<kBf16, 7>(a, grid, s);
-    case 8: return launch_prefill_w<kBf16, 8>(a, grid, s);
-    default: return hipErrorInvalidValue;
+  const int waves = a.group * a.q_tiles;
+  hipError_t e = hipErrorInvalidValue;
+  switch (waves) {
+    case 5: e = launch_prefill_w<kBf16, 5>(a, grid, s); break;
+    case 6: e = launch_prefill_w<kBf16, 6>(a, grid, s); break;
+    case 7: e = launch_prefill_w<kBf16, 7>(a, grid, s); break;
+    case 8: e = launch_prefill_w<kBf16, 8>(a, grid, s); break;
   }
+  if (e != hipSuccess || a.max_tiles == 0) return e;
+  // Units are cut only where two cuts of all of them fit the workspace.
+  hipLaunchKernelGGL(paged_prefill_combine<kBf16>, dim3(unsigned(a.max_tiles / 2), unsigned(waves)), dim3(64 * (kD / 32)), 0, s,
+                     a, waves);
+  return hipGetLastError();
 }
+
+// Tiles of a workspace that lets a call's units be cut over their keys; 0
+// where they would not be: 512 workgroups or more fill the chip without, and
+// a table of fewer than 32 key blocks a sequence (half a unit's time at 4
+// cuts) gains less than the combine's launch costs.
+int64_t prefill_tiles(int group, int n_kv_heads, int n_seqs, int max_q_len, int64_t max_keys) {
+  const int wg_q = kQB * prefill_q_tiles(group);
+  const int64_t n_wg = (int64_t(max_q_len) + wg_q - 1) / wg_q * n_kv_heads * n_seqs;
+  if (n_seqs > kOrderSeqs || n_wg == 0 || n_wg >= 512 || max_keys < 32 * kKB) return 0;
+  return std::min<int64_t>(kMaxTiles, n_wg * kMaxCuts);
+}
+constexpr int64_t kTileWaveBytes = 64 * (16 * 16 + 8);  // a wave's O^T registers and (m, l)
 }  // namespace
+
+extern "C" size_t it_paged_prefill_workspace(int32_t n_heads, int32_t n_kv_heads, int32_t n_seqs, int32_t max_q_len,
+                                             int32_t max_blocks, int32_t block_size) {
+  if (n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || n_seqs <= 0 || max_q_len <= 0 || max_blocks <= 0 ||
+      block_size <= 0)
+    return 0;
+  const int group = n_heads / n_kv_heads;
+  if (group > kMaxGroup) return 0;
+  const int64_t tiles = prefill_tiles(group, n_kv_heads, n_seqs, max_q_len, int64_t(max_blocks) * block_size);
+  return size_t(tiles * group * prefill_q_tiles(group) * kTileWaveBytes);
+}
 
 extern "C" int32_t it_paged_prefill(const it_kv_cache* c, const void* q, int32_t q_dtype, int32_t n_heads,
                                     const int32_t* cu_q, int32_t max_q_len, const int32_t* block_tables,
                                     int32_t max_blocks, const int32_t* ctx_lens, int32_t n_seqs, float scale,
                                     int32_t causal, void* out, int32_t out_dtype, void* stream) {
+  return it_paged_prefill_ws(c, q, q_dtype, n_heads, cu_q, max_q_len, block_tables, max_blocks, ctx_lens, n_seqs, scale,
+                             causal, nullptr, 0, out, out_dtype, stream);
+}
+
+extern "C" int32_t it_paged_prefill_ws(const it_kv_cache* c, const void* q, int32_t q_dtype, int32_t n_heads,
+                                    const int32_t* cu_q, int32_t max_q_len, const int32_t* block_tables,
+                                    int32_t max_blocks, const int32_t* ctx_lens, int32_t n_seqs, float scale,
+                                    int32_t causal, void* ws, size_t ws_bytes, void* out, int32_t out_dtype,
+                                    void* stream) {
   const char* who = "it_paged_prefill";
   if (!c) return fail(IT_INVALID_INPUT, "%s: cache is NULL", who);
   if (int32_t rc = one_layer(c, who)) return rc;
@@ -824,7 +977,18 @@ extern "C" int32_t it_paged_prefill(const it_kv_cache* c, const void* q, int32_t
   a.n_seqs = n_seqs;
   const int64_t n_wg = int64_t(a.n_qb) * c->n_kv_heads * n_seqs;
   if (n_wg > INT32_MAX) return fail(IT_INVALID_INPUT, "%s: %lld workgroups (max 2^31 - 1)", who, (long long)n_wg);
-  const dim3 grid(static_cast<unsigned>(n_wg), 1u, 1u);
+  dim3 grid(static_cast<unsigned>(n_wg), 1u, 1u);
+  if (ws) {
+    if (reinterpret_cast<uintptr_t>(ws) & 255u) return fail(IT_INVALID_INPUT, "%s: ws must be 256-byte aligned", who);
+    const int64_t tiles = prefill_tiles(group, c->n_kv_heads, n_seqs, max_q_len, int64_t(max_blocks) << c->log2_bs);
+    const int64_t waves = int64_t(group) * a.q_tiles;
+    if (ws_bytes < size_t(tiles * waves * kTileWaveBytes))
+      return fail(IT_INVALID_INPUT, "%s: workspace %zu < %zu bytes", who, ws_bytes, size_t(tiles * waves * kTileWaveBytes));
+    a.max_tiles = int(tiles);
+    a.ws_o = static_cast<float4*>(ws);
+    a.ws_ml = reinterpret_cast<float2*>(a.ws_o + tiles * waves * 16 * 64);
+    if (tiles > n_wg) grid.x = unsigned(tiles);
+  }
   int dev = -1;
   (void)hipGetDevice(&dev);
   if (dev != c->device) (void)hipSetDevice(c->device);

@@ -261,10 +261,13 @@ class PagedKvCache:
             scale = 1.0 / math.sqrt(D)
         if out is None:
             out = torch.empty(q.shape, dtype=out_dtype or q.dtype, device=q.device)
-        check(lib.it_paged_prefill(self._h, _ptr(q), torch_dtype_id(q.dtype), n_heads, _ptr(cu_q), max_q_len,
-                                   _ptr(block_tables), block_tables.shape[1], _ptr(ctx_lens), ctx_lens.numel(),
-                                   C.c_float(scale), int(bool(causal)), _ptr(out), torch_dtype_id(out.dtype),
-                                   stream_handle(self.device)))
+        n_seqs, max_blocks = ctx_lens.numel(), block_tables.shape[1]
+        need = lib.it_paged_prefill_workspace(n_heads, self.n_kv_heads, n_seqs, max_q_len, max_blocks, self.block_size)
+        ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+        check(lib.it_paged_prefill_ws(self._h, _ptr(q), torch_dtype_id(q.dtype), n_heads, _ptr(cu_q), max_q_len,
+                                      _ptr(block_tables), max_blocks, _ptr(ctx_lens), n_seqs, C.c_float(scale),
+                                      int(bool(causal)), _ptr(ws), need, _ptr(out), torch_dtype_id(out.dtype),
+                                      stream_handle(self.device)))
         return out
 
     def __del__(self):

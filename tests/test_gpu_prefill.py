@@ -189,13 +189,13 @@ def test_prefill_config3_rows():
         assert np.all(o <= up + 1e-4) and np.all(o >= dn - 1e-4), f"config3 seq {s}: outside the V hull"
 
 
-@pytest.mark.parametrize("n_seqs,hq,hkv,causal", [(2, 7, 1, True), (63, 8, 1, True), (64, 4, 2, False), (65, 8, 1, True),
-                                                  (256, 8, 1, True), (257, 8, 1, True)])
+@pytest.mark.parametrize("n_seqs,hq,hkv,causal", [(2, 7, 1, True), (24, 8, 1, True), (25, 8, 1, True), (63, 8, 1, True),
+                                                  (64, 4, 2, False), (65, 8, 1, True)])
 def test_prefill_unit_order_ragged(n_seqs, hq, hkv, causal):
-    """Workgroups find their unit in the longest-first order over 64-sequence
-    chunks (up to 256 sequences; more take ids in pair order): batches at the
-    chunks' edges, with empty chunks, chunk lengths of one row, whole prompts
-    and long cached prefixes.  Every row against the oracle, so every unit is
+    """Workgroups find their unit in the longest-first order over up to 64
+    sequences (searched one way up to 24, another way past them; more than 64
+    take ids in pair order): batches at those edges, with empty chunks, chunk
+    lengths of one row, whole prompts and long cached prefixes.  Every row against the oracle, so every unit is
     computed, and by nobody else (a unit missed leaves its rows unwritten)."""
     rng = np.random.RandomState(n_seqs)
     q_lens = rng.choice([0, 1, 31, 32, 33, 65, 100], n_seqs)
@@ -206,3 +206,34 @@ def test_prefill_unit_order_ragged(n_seqs, hq, hkv, causal):
     out, scale = _run(dev, tables, ctx, cu, q, td, hq, causal=causal)
     want = ref.prefill(widen(q, orc.BF16), hq, cu, tables, ctx, scale, causal=causal)
     assert_close(from_dev(out), want, RTOL, ATOL, what=f"prefill order n_seqs={n_seqs}")
+
+
+@pytest.mark.parametrize("dt,hq,hkv,ctx,q_lens,causal", [
+    (orc.BF16, 8, 2, [2100], [70], True),          # one long context, few rows: 8 cuts
+    (orc.F16, 7, 1, [4096, 130], [33, 1], True),   # 7 waves; a unit too short to cut beside long ones
+    (orc.BF16, 5, 1, [2049, 0, 3000], [1, 0, 129], True),  # 5 waves, an empty sequence, the diagonal inside the last cut
+    (orc.BF16, 2, 2, [2111], [300], False),        # 8 query tiles a workgroup, every key visible
+    (orc.BF16, 8, 1, [1100, 1023], [64, 64], True),  # at the edge: 17 and 16 key blocks
+])
+def test_prefill_units_cut_over_keys(dt, hq, hkv, ctx, q_lens, causal):
+    """Launches of few units divide each unit's key blocks among several
+    workgroups and merge their partial (m, l, O).  Against the oracle, and
+    against the same call without a workspace (no cuts): the two differ by
+    the rounding of the 16-bit probabilities to different maxima."""
+    import torch
+    from infer_train_amd import lib
+
+    gain = lambda p: 1.0 + (p % 700) / 300.0  # noqa: E731  cuts with different maxima
+    dev, ref, tables, ctx, cu, q, td = _setup(dt, hq, hkv, ctx, q_lens, seed=900 + hq, mb=260, k_gain=gain)
+    need = lib.it_paged_prefill_workspace(hq, hkv, len(ctx), int(max(q_lens)), 260, 16)
+    assert need > 0
+    out, scale = _run(dev, tables, ctx, cu, q, td, hq, causal=causal)
+    want = ref.prefill(widen(q, dt), hq, cu, tables, ctx, scale, causal=causal)
+    got = from_dev(out)
+    assert_close(got, want, RTOL, ATOL, what=f"prefill cut dt={dt} hq={hq}")
+    dq, plain = to_dev(q.view(np.int16), td), torch.empty(q.shape, dtype=torch.float32, device="cuda")
+    dcu, dt_, dctx = to_dev(cu), to_dev(tables), to_dev(ctx)
+    assert lib.it_paged_prefill(dev.handle, dq.data_ptr(), dev.dtype, hq, dcu.data_ptr(), int(max(q_lens)), dt_.data_ptr(),
+                                260, dctx.data_ptr(), len(ctx), scale, int(causal), plain.data_ptr(), 0,
+                                torch.cuda.current_stream().cuda_stream) == 0
+    assert_close(got, from_dev(plain), RTOL, ATOL, what="cut against uncut")
