@@ -408,3 +408,33 @@ def test_append_rope_bad_position_is_latched():
         rows = from_dev(pool).reshape(8, 16, 128 * 4)
         assert np.all(rows[0, 4] == SENTINEL), "a row with an out-of-table position must not be written"
         assert not np.all(rows[0, 3] == SENTINEL)
+
+
+@pytest.mark.parametrize("dt,D,hq,hkv,n,n_dims", [
+    (orc.BF16, 64, 3, 1, 5, 64),     # 4 rows an instruction; 5 rows in all
+    (orc.F16, 128, 9, 3, 1, 96),     # one token, 15 rows, the last 32 dims unrotated
+    (orc.Q8_0, 256, 5, 5, 3, 256),   # a row an instruction, q / k / v borders inside a wave's four
+    (orc.Q4_0, 32, 7, 7, 4, 32),     # 8 rows an instruction
+    (orc.F32, 16, 2, 1, 6, 4),       # the narrowest row taken so: 16 rows an instruction
+    (orc.BF16, 96, 4, 2, 5, 96),     # not a power of two: one vector per lane
+])
+def test_append_rope_row_shapes(dt, D, hq, hkv, n, n_dims):
+    """Head counts that do not fill a wave's rows, every row width, partly
+    rotated rows: pools and rotated q equal the oracle's byte for byte."""
+    from infer_train_amd.kv import RopeTable
+
+    nb, bs = 8, 16
+    dev, ref = _pair(nb, bs, hkv, D, dt)
+    rope = RopeTable(n_dims, 300)
+    rng = np.random.default_rng(D)
+    slots = rng.permutation(nb * bs)[:n].astype(np.int64)
+    if n > 3:
+        slots[2] = -1
+    pos = rng.integers(0, 300, n).astype(np.int32)
+    q, k, v = (orc.normal(70 + i, n * h * D).reshape(n, h, D) for i, h in enumerate((hq, hkv, hkv)))
+    q_rot, k_rot = orc.rope_rows(q, pos, n_dims, D), orc.rope_rows(k, pos, n_dims, D)
+    ref.append(_to_cache_src(k_rot, dt), _to_cache_src(v, dt), slots)
+    q_out = dev.append_rope(rope, to_dev(q), to_dev(k), to_dev(v), to_dev(slots), to_dev(pos))
+    dev.check()
+    _assert_pools(dev, ref, f"append_rope rows dt={dt} D={D}")
+    assert np.array_equal(from_dev(q_out).view(np.uint32), q_rot.view(np.uint32))
