@@ -234,6 +234,89 @@ __global__ __launch_bounds__(kThreads) void kv_append_q8_wide(
   }
 }
 
+// Q4_0 / Q4_1 / Q5_0 / Q5_1 quantise-append with 16-byte stores (head_dim D =
+// 64, 128, 256).  A wave takes 2048 consecutive source floats, 64 groups:
+//  - Loads: eight instructions of 1 KiB, all issued before the first is used.
+//  - Quantise: eight lanes per 32-group (quant_group).
+//  - The groups' nibble bytes and words go through a wave-private LDS stage
+//    (same-wave LDS operations stay in order); lane L then stores group L: its
+//    16 nibble bytes as one vector, its qh word, its d or (d, m).
+// Bound by memory and, near it, by the quantiser's VALU.  4096 tokens of 4 x
+// 256, Q4_0 (38 MB): 8.5 us, 4.5 TB/s (one vector per lane, 4- and 2-byte
+// stores: 12.4 us).  blockIdx.y selects K (0) or V (1).
+template <int DT, int D>
+__global__ __launch_bounds__(kThreads) void kv_append_nib_wide(
+    const float* __restrict__ k, const float* __restrict__ v, char* __restrict__ kpool, char* __restrict__ vpool,
+    const int64_t* __restrict__ slots, int32_t n_rows, int32_t n_chunks, int hkv, int log2_bs, int64_t page_bytes,
+    int64_t n_slots, uint32_t* err) {
+  using N = NibFmt<DT>;
+  constexpr int NG = D / 32;     // groups (and store lanes) per row
+  constexpr int RPW = 2048 / D;  // rows per chunk
+  constexpr int kWaves = kThreads / 64;
+  __shared__ __attribute__((aligned(16))) uint32_t st_q[kWaves][256];
+  __shared__ uint32_t st_m[kWaves][64], st_h[kWaves][N::kQ5 ? 64 : 1];
+  const bool is_v = blockIdx.y != 0;
+  const int lane = int(threadIdx.x & 63u), wave = int(threadIdx.x >> 6);
+  const int log2_hkv = (hkv & (hkv - 1)) == 0 ? __builtin_ctz(unsigned(hkv)) : -1;  // uniform
+  const float* const src = is_v ? v : k;
+  char* const pool = is_v ? vpool : kpool;
+  const int64_t last = int64_t(n_rows) * D - 4;
+  const int32_t stride = int32_t(gridDim.x) * kWaves;
+  for (int32_t c = int32_t(blockIdx.x) * kWaves + wave; c < n_chunks; c += stride) {  // uniform
+    const int32_t row = c * RPW + lane / NG;
+    const int32_t rs = row < n_rows ? row : n_rows - 1;
+    const int32_t tok = log2_hkv >= 0 ? rs >> log2_hkv : rs / hkv;
+    const int64_t sl = slots[tok];
+    const int64_t f0 = int64_t(c) * 2048 + 4 * lane;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    f4 x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)  // past the end a lane re-reads the last four floats; those rows are not stored
+      x[j] = __builtin_nontemporal_load(reinterpret_cast<const f4*>(src + min(f0 + 256 * j, last)));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const QuantGroup q = quant_group<DT>(make_float4(x[j].x, x[j].y, x[j].z, x[j].w), lane & 7);
+      const int g = 8 * j + (lane >> 3);
+      if ((lane & 7) < 4) st_q[wave][4 * g + (lane & 7)] = q.qs;
+      if ((lane & 7) == 0) {
+        st_m[wave][g] = q.meta;
+        if constexpr (N::kQ5) st_h[wave][g] = q.qh;
+      }
+    }
+    const uint4 w = *reinterpret_cast<const uint4*>(&st_q[wave][4 * lane]);
+    const uint32_t meta = st_m[wave][lane];
+    uint32_t qh = 0u;
+    if constexpr (N::kQ5) qh = st_h[wave][lane];
+    if (row < n_rows && sl >= 0) {
+      const int g = lane % NG;
+      const int h = row - tok * hkv;
+      if (sl >= n_slots) {
+        if (g == 0 && h == 0) atomicOr(err, kErrSlot);
+      } else {
+        const int64_t blk = sl >> log2_bs;
+        const int64_t off = sl & ((int64_t(1) << log2_bs) - 1);
+        char* const page = pool + (blk * hkv + h) * page_bytes;
+        st16(page + off * (D / 2) + 16 * g, w);
+        char* const side = page + (int64_t(1) << log2_bs) * (D / 2) + off * (NG * N::kSide);
+        if constexpr (N::kQ5) *reinterpret_cast<uint32_t*>(side + 4 * g) = qh;
+        if constexpr (N::kMin) *reinterpret_cast<uint32_t*>(side + N::meta_off(NG) + 4 * g) = meta;
+        else *reinterpret_cast<uint16_t*>(side + N::meta_off(NG) + 2 * g) = uint16_t(meta);
+      }
+    }
+  }
+}
+
+// Fewest chunks it is used for.  A wave quantises its eight instructions one
+// after another, which costs appends that leave SIMDs idle 1.2 to 2 us (Q4_0 /
+// Q5_1): 256 chunks 4.4 us so against 3.5 a vector per lane, 512 4.6 / 5.8
+// against 4.7 / 5.3, 1024 5.9 (Q4_0) against 7.9.
+constexpr int64_t kWideChunks = 768;
+
+template <int DT>
+auto* nib_wide(int d) {
+  return d == 256 ? kv_append_nib_wide<DT, 256> : d == 128 ? kv_append_nib_wide<DT, 128> : kv_append_nib_wide<DT, 64>;
+}
+
 // ---------------------------------------------------------------------------
 // Gather.  grid.y = sequence; lane = one 16-byte vector of one output row.
 // ---------------------------------------------------------------------------
@@ -686,6 +769,19 @@ extern "C" int32_t it_kv_append(it_kv_cache* c, const void* k, const void* v, in
     hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, s, (const float*)k, (const float*)v, (char*)c->k_pool,
                        (char*)c->v_pool, slots, int32_t(q8_rows), int32_t(groups), c->n_kv_heads, c->log2_bs, c->page_bytes,
                        n_slots, c->err_flag);
+  } else if (quant && c->dtype != IT_Q8_0 && (c->head_dim == 64 || c->head_dim == 128 || c->head_dim == 256) &&
+             q8_rows < (int64_t(1) << 30) && cdiv(q8_rows, 2048 / c->head_dim) >= kWideChunks) {
+    // Chunks of 64 groups, one per wave, up to eight waves per SIMD; larger
+    // appends loop.
+    const int64_t chunks = cdiv(q8_rows, 2048 / c->head_dim);
+    dim3 grid(unsigned(cdiv(std::min<int64_t>(chunks, 8192), kThreads / 64)), 2);
+    auto* kern = c->dtype == IT_Q4_0   ? nib_wide<IT_Q4_0>(c->head_dim)
+                 : c->dtype == IT_Q4_1 ? nib_wide<IT_Q4_1>(c->head_dim)
+                 : c->dtype == IT_Q5_0 ? nib_wide<IT_Q5_0>(c->head_dim)
+                                       : nib_wide<IT_Q5_1>(c->head_dim);
+    hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, s, (const float*)k, (const float*)v, (char*)c->k_pool,
+                       (char*)c->v_pool, slots, int32_t(q8_rows), int32_t(chunks), c->n_kv_heads, c->log2_bs,
+                       c->page_bytes, n_slots, c->err_flag);
   } else if (quant) {
     const int64_t total = int64_t(n_tokens) * c->n_kv_heads * (c->head_dim / 4);
     dim3 grid(unsigned(cdiv(total, kThreads)), 2);

@@ -97,38 +97,37 @@ __device__ __forceinline__ bool q8_fast_scale(float scale) { return scale >= 0x1
 // 127 needs no clamp.  Otherwise (near a tie, or NaN) the IEEE division
 // decides.
 
-// (int8_t)(r) and (uint8_t)(r) as ggml's x86 build computes them: truncate
-// to int32 (NaN and out-of-range give 0x80000000), keep the low byte.
-__device__ __forceinline__ int32_t trunc_i8(float r) {
-  if (!(fabsf(r) < 2147483648.0f)) return 0;
-  return int32_t(int8_t(int32_t(r)));
+// A value's code: (int8_t)(r) (Q5_1: (uint8_t)(r)) as ggml's x86 build
+// computes it (truncate; NaN and what int32 cannot hold give a low byte of 0),
+// at most `top`.  r = x id + half + 0.5 with |x| <= |max| and id = 1 / (max /
+// -half), or (x - min) id + 0.5 with id = 1 / ((max - min) / top): when id is
+// finite d is at least 2^-128, rounded by 2^-22 at most, so r lies in (0, 2
+// half + 1); else the product is infinite or NaN.  So r is a small positive
+// number or the code is 0, and an unsigned convert and one bound say which.
+__device__ __forceinline__ uint32_t quant_code(float r, uint32_t top) {
+  return min(uint32_t(r < 64.0f ? r : 0.0f), top);  // NaN fails the compare; r > -1
 }
-__device__ __forceinline__ int32_t trunc_u8(float r) {
-  if (!(fabsf(r) < 2147483648.0f)) return 0;
-  return int32_t(uint8_t(int32_t(r)));
+
+// Steps of a reduction over an 8-lane group in which the lower lane wins
+// ties: f(DPP control, whether this lane's partner is the lower one).
+template <class F>
+__device__ __forceinline__ void group8_steps(int l8, F&& f) {
+  f(std::integral_constant<int, kDppQuadXor1>{}, (l8 & 1) != 0);
+  f(std::integral_constant<int, kDppQuadXor2>{}, (l8 & 2) != 0);
+  f(std::integral_constant<int, kDppHalfMirror>{}, (l8 & 4) != 0);
 }
-// Q4's min(15, (int8_t)r), low byte.
-__device__ __forceinline__ uint32_t q4_nibble(float r) { return uint32_t(min(trunc_i8(r), 15)) & 0xFFu; }
 
 // The value of largest magnitude in an 8-lane group of four floats per lane
-// (equal magnitudes: the lower element index; NaN never wins; none: 0).
+// (equal magnitudes: the lower element index; NaN never wins; none: 0).  The
+// winner is carried, not its index: each step knows which lane is lower.
 __device__ __forceinline__ float group_absmax_first(const float (&xs)[4], int l8) {
-  float am = 0.0f, mx = 0.0f;
-  int im = 32;
+  float mx = 0.0f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float a = fabsf(xs[e]);
-    if (am < a) am = a, mx = xs[e], im = 4 * l8 + e;
-  }
-  auto step = [&](auto ctrl) {
-    constexpr int C = decltype(ctrl)::value;
-    const float a2 = dpp_f<C>(am), m2 = dpp_f<C>(mx);
-    const int i2 = __builtin_amdgcn_mov_dpp(im, C, 0xF, 0xF, true);
-    if (a2 > am || (a2 == am && i2 < im)) am = a2, mx = m2, im = i2;
-  };
-  step(std::integral_constant<int, kDppQuadXor1>{});
-  step(std::integral_constant<int, kDppQuadXor2>{});
-  step(std::integral_constant<int, kDppHalfMirror>{});
+  for (int e = 0; e < 4; ++e) mx = fabsf(xs[e]) > fabsf(mx) ? xs[e] : mx;
+  group8_steps(l8, [&](auto ctrl, bool low) {
+    const float m2 = dpp_f<decltype(ctrl)::value>(mx);
+    if (fabsf(m2) > fabsf(mx) || (low && fabsf(m2) == fabsf(mx))) mx = m2;
+  });
   return mx;
 }
 
@@ -136,23 +135,16 @@ __device__ __forceinline__ float group_absmax_first(const float (&xs)[4], int l8
 // first of equal values stays; FLT_MAX / -FLT_MAX when every element is NaN).
 __device__ __forceinline__ void group_minmax(const float (&xs)[4], int l8, float& mn, float& mx) {
   mn = FLT_MAX, mx = -FLT_MAX;
-  int imn = 32, imx = 32;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    if (xs[e] < mn) mn = xs[e], imn = 4 * l8 + e;
-    if (xs[e] > mx) mx = xs[e], imx = 4 * l8 + e;
+    mn = xs[e] < mn ? xs[e] : mn;
+    mx = xs[e] > mx ? xs[e] : mx;
   }
-  auto step = [&](auto ctrl) {
-    constexpr int C = decltype(ctrl)::value;
-    const float mn2 = dpp_f<C>(mn), mx2 = dpp_f<C>(mx);
-    const int imn2 = __builtin_amdgcn_mov_dpp(imn, C, 0xF, 0xF, true);
-    const int imx2 = __builtin_amdgcn_mov_dpp(imx, C, 0xF, 0xF, true);
-    if (mn2 < mn || (mn2 == mn && imn2 < imn)) mn = mn2, imn = imn2;
-    if (mx2 > mx || (mx2 == mx && imx2 < imx)) mx = mx2, imx = imx2;
-  };
-  step(std::integral_constant<int, kDppQuadXor1>{});
-  step(std::integral_constant<int, kDppQuadXor2>{});
-  step(std::integral_constant<int, kDppHalfMirror>{});
+  group8_steps(l8, [&](auto ctrl, bool low) {
+    const float mn2 = dpp_f<decltype(ctrl)::value>(mn), mx2 = dpp_f<decltype(ctrl)::value>(mx);
+    if (mn2 < mn || (low && mn2 == mn)) mn = mn2;
+    if (mx2 > mx || (low && mx2 == mx)) mx = mx2;
+  });
 }
 
 // OR of a word over an 8-lane group.
@@ -223,7 +215,7 @@ __device__ __forceinline__ QuantGroup quant_group(float4 x, int l8) {
     const float d = group_absmax_first(xs, l8) / -8.0f;
     const float id = d != 0.0f ? 1.0f / d : 0.0f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out.qs |= q4_nibble(mul_rn(xs[e], id) + 8.5f) << (8 * e);
+    for (int e = 0; e < 4; ++e) out.qs |= quant_code(mul_rn(xs[e], id) + 8.5f, 15u) << (8 * e);
     out.meta = f16_bits_rne(d);
   } else if constexpr (DT == IT_Q4_1) {
     float mn, mx;
@@ -231,16 +223,16 @@ __device__ __forceinline__ QuantGroup quant_group(float4 x, int l8) {
     const float d = (mx - mn) / 15.0f;
     const float id = d != 0.0f ? 1.0f / d : 0.0f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out.qs |= q4_nibble(mul_rn(xs[e] - mn, id) + 0.5f) << (8 * e);
+    for (int e = 0; e < 4; ++e) out.qs |= quant_code(mul_rn(xs[e] - mn, id) + 0.5f, 15u) << (8 * e);
     out.meta = f16_bits_rne(d) | (f16_bits_rne(mn) << 16);
   } else {
     static_assert(DT == IT_Q5_0 || DT == IT_Q5_1, "Q8_0, Q4_0, Q4_1, Q5_0 or Q5_1");
-    int32_t q[4];
+    uint32_t q[4];
     if constexpr (DT == IT_Q5_0) {
       const float d = group_absmax_first(xs, l8) / -16.0f;
       const float id = d != 0.0f ? 1.0f / d : 0.0f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) q[e] = min(trunc_i8(mul_rn(xs[e], id) + 16.5f), 31);
+      for (int e = 0; e < 4; ++e) q[e] = quant_code(mul_rn(xs[e], id) + 16.5f, 31u);
       out.meta = f16_bits_rne(d);
     } else {
       float mn, mx;
@@ -248,14 +240,14 @@ __device__ __forceinline__ QuantGroup quant_group(float4 x, int l8) {
       const float d = (mx - mn) / 31.0f;
       const float id = d != 0.0f ? 1.0f / d : 0.0f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) q[e] = trunc_u8(mul_rn(xs[e] - mn, id) + 0.5f);
+      for (int e = 0; e < 4; ++e) q[e] = quant_code(mul_rn(xs[e] - mn, id) + 0.5f, 31u);
       out.meta = f16_bits_rne(d) | (f16_bits_rne(mn) << 16);
     }
     uint32_t hb = 0u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      out.qs |= (uint32_t(q[e]) & 0xFu) << (8 * e);
-      hb |= ((uint32_t(q[e]) >> 4) & 1u) << e;
+      out.qs |= (q[e] & 0xFu) << (8 * e);
+      hb |= (q[e] >> 4) << e;
     }
     out.qh = group_or8(hb << (4 * l8));
   }

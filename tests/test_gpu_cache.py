@@ -438,3 +438,36 @@ def test_append_rope_row_shapes(dt, D, hq, hkv, n, n_dims):
     dev.check()
     _assert_pools(dev, ref, f"append_rope rows dt={dt} D={D}")
     assert np.array_equal(from_dev(q_out).view(np.uint32), q_rot.view(np.uint32))
+
+
+@pytest.mark.parametrize("dt,D,hkv,n", [
+    (orc.Q4_0, 256, 3, 1), (orc.Q4_1, 64, 2, 33), (orc.Q5_0, 128, 5, 7), (orc.Q5_1, 256, 1, 8),
+    (orc.Q4_0, 64, 5, 4908), (orc.Q4_0, 64, 5, 4915),  # either side of the wide kernel's smallest append
+    (orc.Q4_1, 128, 3, 4097), (orc.Q5_0, 256, 1, 6140), (orc.Q5_1, 128, 4, 4000), (orc.Q5_0, 64, 8, 3073),
+    (orc.Q4_1, 256, 8, 8201)])                         # more chunks than waves in one launch
+def test_append_nibble_chunks_and_scales(dt, D, hkv, n):
+    """Both nibble appends (a vector per lane; 64 groups a wave) with whole
+    chunks and parts of one, on groups of every
+    magnitude: scales from fp32 subnormals (1 / d overflows) to near the
+    largest float (max - min overflows), equal magnitudes of both signs,
+    signed zeros, NaN and inf elements.  Bytes equal the oracle's."""
+    bs = 16
+    nb = (n + bs - 1) // bs + 3
+    rng = np.random.default_rng(n * D + int(dt))
+    x = rng.standard_normal((2, n * hkv * D // 32, 32)).astype(np.float32)
+    scale = np.float32(10.0) ** rng.uniform(-46, 38.2, (2, x.shape[1], 1))
+    x = np.where(rng.random((2, x.shape[1], 1)) < 0.5, x, x * scale).astype(np.float32)
+    pick = lambda p: rng.random(x.shape) < p  # noqa: E731
+    tie = np.abs(x).max(-1, keepdims=True)
+    x = np.where(pick(0.02), np.where(pick(0.5), tie, -tie), x).astype(np.float32)
+    for value, p in ((0.0, 0.02), (-0.0, 0.02), (np.nan, 0.002), (np.inf, 0.001), (-np.inf, 0.001), (3.4028235e38, 0.0005)):
+        x[pick(p)] = value
+    x[:, ::17] = np.where(pick(0.5)[:, ::17], np.float32(0.0), np.float32(-0.0))  # all-zero groups
+    k, v = (a.reshape(n, hkv, D).copy() for a in x)
+    dev, ref = _pair(nb, bs, hkv, D, dt)
+    slots = orc.permutation(D + n, nb * bs)[:n].copy()
+    if n > 2:
+        slots[1] = -1
+    ref.append(k, v, slots)
+    dev.append(to_dev(k), to_dev(v), to_dev(slots))
+    _assert_pools(dev, ref, f"append nibble dt={dt} D={D} n={n}")
