@@ -357,71 +357,37 @@ __global__ __launch_bounds__(kThreads) void kv_gather_vec(
   st16(vout + dst, ld16_nt(vpool + src));
 }
 
-// Q8_0 gather: lane = one 32-element group, written as a packed 34-byte
-// BlockQ8_0 record {u16 d; i8 qs[32]} (types.rs:34-41).
-__global__ __launch_bounds__(kThreads) void kv_gather_q8_0(
-    const char* __restrict__ kpool, const char* __restrict__ vpool, const int32_t* __restrict__ bt,
-    int max_blocks, const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ start_pos,
-    const int64_t* __restrict__ cu_out, int hkv, int d, int log2_bs, int64_t page_bytes,
-    int64_t num_blocks, char* __restrict__ kout, char* __restrict__ vout, uint32_t* err) {
-  const int b = blockIdx.y;
-  const int st = start_pos ? start_pos[b] : 0;
-  const int n = ctx_lens[b] - st;
-  if (st < 0) {  // skipped and latched
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, kErrStart);
-    return;
-  }
-  if (n <= 0) return;
-  const int ng = d >> 5;
-  const int64_t gid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (gid >= int64_t(hkv) * n * ng) return;
-  const int g = int(gid % ng);
-  const int64_t r = gid / ng;
-  const int i = int(r % n);
-  const int h = int(r / n);
-  const int pos = st + i;
-  const int lb = pos >> log2_bs;
-  if (lb >= max_blocks) {
-    atomicOr(err, kErrTable);
-    return;
-  }
-  const int blk = bt[int64_t(b) * max_blocks + lb];
-  if (blk < 0 || blk >= num_blocks) {
-    atomicOr(err, kErrBlock);
-    return;
-  }
-  const int64_t bs = int64_t(1) << log2_bs;
-  const int64_t off = pos & (bs - 1);
-  const int64_t rec = ((cu_out[b] * hkv + int64_t(h) * n + i) * ng + g) * 34;
-  for (int which = 0; which < 2; ++which) {
-    const char* page = (which ? vpool : kpool) + (int64_t(blk) * hkv + h) * page_bytes;
-    const uint4 q0 = ld16(page + off * d + g * 32);
-    const uint4 q1 = ld16(page + off * d + g * 32 + 16);
-    const uint16_t dd = *reinterpret_cast<const uint16_t*>(page + bs * d + (off * ng + g) * 2);
-    uint16_t* o = reinterpret_cast<uint16_t*>((which ? vout : kout) + rec);  // 2-byte aligned
-    o[0] = dd;
-    const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      o[1 + 2 * j] = uint16_t(w[j] & 0xFFFFu);
-      o[2 + 2 * j] = uint16_t(w[j] >> 16);
-    }
-  }
-}
-
-// Q4_0 / Q4_1 / Q5_0 / Q5_1 gather: lane = one 32-element group, written as
-// a packed ggml record {meta; [qh;] qs[16]}: BlockQ4_0 {u16 d} (18 bytes,
-// types.rs:15-22), BlockQ4_1 {u16 d; u16 m} (20, types.rs:24-32),
-// block_q5_0 {u16 d; u8 qh[4]} (22) and block_q5_1 {u16 d; u16 m; u8
-// qh[4]} (24).  Records of 18 and 22 bytes are 2-byte aligned, so the
-// stores are 16-bit.
+// Quantised gather: lane = one 32-element group, written as a packed record:
+// BlockQ8_0 {u16 d; i8 qs[32]} (34 bytes, types.rs:34-41), BlockQ4_0 {u16 d;
+// u8 qs[16]} (18, types.rs:15-22), BlockQ4_1 {u16 d; u16 m; qs} (20,
+// types.rs:24-32), ggml's block_q5_0 {u16 d; u8 qh[4]; qs} (22) and block_q5_1
+// {u16 d; u16 m; u8 qh[4]; qs} (24).  A sequence's records of one KV head
+// follow one another, so a wave's 64 are one run of a multiple of 128 bytes:
+// they are packed in a wave-private LDS stage (same-wave LDS operations stay
+// in order) and stored as 16-byte vectors, or 4- or 2-byte ones where the run
+// starts unaligned (groups of a row that is not a multiple of 8 records).
+// blockIdx.x holds (KV head, 256 groups); blockIdx.y is the sequence.
+// Bound by memory: 4 sequences of 4096 to 16384 tokens, 4 x 256, Q8_0 (194
+// MB): 41.0 us, 4.7 TB/s (2-byte stores straight to the records: 46.9 us);
+// small gathers wait for the stage (1.4 MB of 8 sequences: 3.3 us against 2.9).
 template <int DT>
-__global__ __launch_bounds__(kThreads) void kv_gather_nib(
+struct GatherRec {
+  static constexpr int kBytes = NibFmt<DT>::kRecord;
+};
+template <>
+struct GatherRec<IT_Q8_0> {
+  static constexpr int kBytes = IT_BLOCK_Q8_0_BYTES;
+};
+
+template <int DT>
+__global__ __launch_bounds__(kThreads) void kv_gather_quant(
     const char* __restrict__ kpool, const char* __restrict__ vpool, const int32_t* __restrict__ bt,
     int max_blocks, const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ start_pos,
     const int64_t* __restrict__ cu_out, int hkv, int d, int log2_bs, int64_t page_bytes,
-    int64_t num_blocks, char* __restrict__ kout, char* __restrict__ vout, uint32_t* err) {
-  using N = NibFmt<DT>;
+    int64_t num_blocks, unsigned head_wgs, char* __restrict__ kout, char* __restrict__ vout, uint32_t* err) {
+  constexpr int REC = GatherRec<DT>::kBytes;
+  constexpr bool kQ8 = DT == IT_Q8_0;
+  __shared__ __attribute__((aligned(16))) char stage[kThreads / 64][2][64 * REC];
   const int b = blockIdx.y;
   const int st = start_pos ? start_pos[b] : 0;
   const int n = ctx_lens[b] - st;
@@ -429,55 +395,124 @@ __global__ __launch_bounds__(kThreads) void kv_gather_nib(
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, kErrStart);
     return;
   }
-  if (n <= 0) return;
-  const int ng = d >> 5;
-  const int64_t gid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (gid >= int64_t(hkv) * n * ng) return;
-  const int g = int(gid % ng);
-  const int64_t r = gid / ng;
-  const int i = int(r % n);
-  const int h = int(r / n);
-  const int pos = st + i;
-  const int lb = pos >> log2_bs;
+  const unsigned h = blockIdx.x / head_wgs;
+  const int ng = d >> 5, lane = int(threadIdx.x & 63);
+  const int64_t total = n > 0 ? int64_t(n) * ng : 0;  // the head's groups
+  const int64_t wave0 = int64_t(blockIdx.x - h * head_wgs) * kThreads + (threadIdx.x & ~63u);
+  if (wave0 >= total) return;  // uniform in the wave
+  const int64_t idx = wave0 + lane;
+  const bool live = idx < total;
+  // Group g of token i (32-bit division wherever the head's groups allow it).
+  const int64_t at = live ? idx : total - 1;
+  const int64_t i = (total >> 32) ? at / ng : int64_t(uint32_t(at) / uint32_t(ng));
+  const int g = int(at - i * ng);
+  const int64_t pos = int64_t(st) + i;
+  const int64_t lb = pos >> log2_bs;
+  int blk = -1;
   if (lb >= max_blocks) {
     atomicOr(err, kErrTable);
-    return;
+  } else {
+    blk = bt[int64_t(b) * max_blocks + lb];
+    if (blk < 0 || blk >= num_blocks) {
+      atomicOr(err, kErrBlock);
+      blk = -1;
+    }
   }
-  const int blk = bt[int64_t(b) * max_blocks + lb];
-  if (blk < 0 || blk >= num_blocks) {
-    atomicOr(err, kErrBlock);
-    return;
-  }
-  const int64_t bs = int64_t(1) << log2_bs;
-  const int64_t off = pos & (bs - 1);
-  const int64_t rec = ((cu_out[b] * hkv + int64_t(h) * n + i) * ng + g) * N::kRecord;
-  for (int which = 0; which < 2; ++which) {
-    const char* page = (which ? vpool : kpool) + (int64_t(blk) * hkv + h) * page_bytes;
-    const uint4 q = ld16(page + off * (d >> 1) + g * 16);
-    const char* side = page + bs * (d >> 1) + off * (ng * N::kSide);
-    uint16_t w[N::kRecord / 2];
-    int k = 0;
-    if constexpr (N::kMin) {
-      const uint32_t dm = *reinterpret_cast<const uint32_t*>(side + N::meta_off(ng) + 4 * g);
-      w[k++] = uint16_t(dm & 0xFFFFu);
-      w[k++] = uint16_t(dm >> 16);
+  const bool found = blk >= 0;
+  const int64_t bs = int64_t(1) << log2_bs, off = pos & (bs - 1);
+  const int64_t page = (int64_t(found ? blk : 0) * hkv + h) * page_bytes;
+  // Both pools' words first, then the stage.
+  constexpr int QB = kQ8 ? 32 : 16;  // main-plane bytes of a group
+  uint4 q[2][QB / 16];
+  uint32_t meta[2], qh[2];
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const char* const pg = (w ? vpool : kpool) + page;
+    const char* const main = pg + (off * ng + g) * QB;
+    const char* const side = pg + bs * ng * QB;
+#pragma unroll
+    for (int c = 0; c < QB / 16; ++c) q[w][c] = ld16(main + 16 * c);
+    qh[w] = 0u;
+    if constexpr (kQ8) {
+      meta[w] = *reinterpret_cast<const uint16_t*>(side + (off * ng + g) * 2);
     } else {
-      w[k++] = *reinterpret_cast<const uint16_t*>(side + N::meta_off(ng) + 2 * g);
+      using N = NibFmt<DT>;
+      const char* const row = side + off * (ng * N::kSide);
+      if constexpr (N::kMin) meta[w] = *reinterpret_cast<const uint32_t*>(row + N::meta_off(ng) + 4 * g);
+      else meta[w] = *reinterpret_cast<const uint16_t*>(row + N::meta_off(ng) + 2 * g);
+      if constexpr (N::kQ5) qh[w] = *reinterpret_cast<const uint32_t*>(row + 4 * g);
     }
-    if constexpr (N::kQ5) {
-      const uint32_t qh = *reinterpret_cast<const uint32_t*>(side + 4 * g);
-      w[k++] = uint16_t(qh & 0xFFFFu);
-      w[k++] = uint16_t(qh >> 16);
-    }
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+  }
+  const int n_rec = int(min(int64_t(64), total - wave0));
+  const int64_t rec0 = ((cu_out[b] * hkv + int64_t(h) * n) * ng + wave0) * REC;
+  const bool whole = __builtin_amdgcn_ballot_w64(live && !found) == 0;  // no record of the wave is skipped
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      w[k++] = uint16_t(qw[j] & 0xFFFFu);
-      w[k++] = uint16_t(qw[j] >> 16);
+  for (int w = 0; w < 2; ++w) {
+    char* const sg = stage[threadIdx.x >> 6][w];
+    uint16_t* o = reinterpret_cast<uint16_t*>(sg + lane * REC);
+    auto put = [&](uint32_t x) {
+      o[0] = uint16_t(x & 0xFFFFu);
+      o[1] = uint16_t(x >> 16);
+      o += 2;
+    };
+    if constexpr (kQ8) {
+      *o++ = uint16_t(meta[w]);
+    } else {
+      if constexpr (NibFmt<DT>::kMin) put(meta[w]);
+      else *o++ = uint16_t(meta[w]);
+      if constexpr (NibFmt<DT>::kQ5) put(qh[w]);
     }
-    uint16_t* o = reinterpret_cast<uint16_t*>((which ? vout : kout) + rec);
 #pragma unroll
-    for (int j = 0; j < N::kRecord / 2; ++j) o[j] = w[j];
+    for (int c = 0; c < QB / 16; ++c) {
+      put(q[w][c].x);
+      put(q[w][c].y);
+      put(q[w][c].z);
+      put(q[w][c].w);
+    }
+  }
+  const char* const sk = stage[threadIdx.x >> 6][0];
+  const char* const sv = stage[threadIdx.x >> 6][1];
+  char* const ok = kout + rec0;
+  char* const ov = vout + rec0;
+  // The wave's runs in pieces of sizeof(unit); a last shorter one in 2-byte ones.
+  auto copy = [&](auto unit) {
+    using U = decltype(unit);
+    constexpr int kPieces = (64 * REC / int(sizeof(U)) + 63) / 64;  // of a lane, in a whole run
+    const int bytes = n_rec * REC, n_u = bytes / int(sizeof(U));
+    U xk[kPieces], xv[kPieces];
+#pragma unroll
+    for (int c = 0; c < kPieces; ++c) {
+      const int p = min(lane + 64 * c, 64 * REC / int(sizeof(U)) - 1);
+      xk[c] = reinterpret_cast<const U*>(sk)[p];
+      xv[c] = reinterpret_cast<const U*>(sv)[p];
+    }
+#pragma unroll
+    for (int c = 0; c < kPieces; ++c) {
+      const int p = lane + 64 * c;
+      if (p < n_u) {
+        reinterpret_cast<U*>(ok)[p] = xk[c];
+        reinterpret_cast<U*>(ov)[p] = xv[c];
+      }
+    }
+    const int p = n_u * int(sizeof(U)) + 2 * lane;
+    if (p < bytes) {
+      *reinterpret_cast<uint16_t*>(ok + p) = *reinterpret_cast<const uint16_t*>(sk + p);
+      *reinterpret_cast<uint16_t*>(ov + p) = *reinterpret_cast<const uint16_t*>(sv + p);
+    }
+  };
+  const uintptr_t a = reinterpret_cast<uintptr_t>(ok) | reinterpret_cast<uintptr_t>(ov);  // uniform
+  if (!whole) {  // a lane whose block is out of range leaves its record as it was
+    if (live && found)
+      for (int p = lane * REC; p < lane * REC + REC; p += 2) {
+        *reinterpret_cast<uint16_t*>(ok + p) = *reinterpret_cast<const uint16_t*>(sk + p);
+        *reinterpret_cast<uint16_t*>(ov + p) = *reinterpret_cast<const uint16_t*>(sv + p);
+      }
+  } else if ((a & 15) == 0) {
+    copy(uint4{});
+  } else if ((a & 3) == 0) {
+    copy(uint32_t{});
+  } else {
+    copy(uint16_t{});
   }
 }
 
@@ -830,17 +865,17 @@ extern "C" int32_t it_kv_gather(const it_kv_cache* c, const int32_t* bt, int32_t
   DeviceGuard g(c->device);
   hipStream_t s = (hipStream_t)stream;
   if (is_quant(c->dtype)) {
-    const int64_t per_seq = int64_t(c->n_kv_heads) * max_tokens * (c->head_dim / 32);
-    dim3 grid(unsigned(cdiv(per_seq, kThreads)), unsigned(n_seqs));
-    auto* kern = c->dtype == IT_Q8_0   ? kv_gather_q8_0
-                 : c->dtype == IT_Q4_0 ? kv_gather_nib<IT_Q4_0>
-                 : c->dtype == IT_Q4_1 ? kv_gather_nib<IT_Q4_1>
-                 : c->dtype == IT_Q5_0 ? kv_gather_nib<IT_Q5_0>
-                                       : kv_gather_nib<IT_Q5_1>;
+    const int64_t head_wgs = cdiv(int64_t(max_tokens) * (c->head_dim / 32), kThreads);
+    dim3 grid(unsigned(head_wgs * c->n_kv_heads), unsigned(n_seqs));
+    auto* kern = c->dtype == IT_Q8_0   ? kv_gather_quant<IT_Q8_0>
+                 : c->dtype == IT_Q4_0 ? kv_gather_quant<IT_Q4_0>
+                 : c->dtype == IT_Q4_1 ? kv_gather_quant<IT_Q4_1>
+                 : c->dtype == IT_Q5_0 ? kv_gather_quant<IT_Q5_0>
+                                       : kv_gather_quant<IT_Q5_1>;
     hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, s,
                        (const char*)c->k_pool, (const char*)c->v_pool,
                        bt, max_blocks, ctx_lens, start_pos, cu_out, c->n_kv_heads, c->head_dim, c->log2_bs,
-                       c->page_bytes, c->num_blocks, (char*)k_out, (char*)v_out, c->err_flag);
+                       c->page_bytes, c->num_blocks, unsigned(head_wgs), (char*)k_out, (char*)v_out, c->err_flag);
   } else {
     if (!aligned16(k_out) || !aligned16(v_out)) return fail(IT_INVALID_INPUT, "it_kv_gather: outputs must be 16-byte aligned");
     const int row_vecs = int(c->head_dim * dtype_bytes(c->dtype) / 16);

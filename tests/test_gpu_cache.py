@@ -471,3 +471,50 @@ def test_append_nibble_chunks_and_scales(dt, D, hkv, n):
     ref.append(k, v, slots)
     dev.append(to_dev(k), to_dev(v), to_dev(slots))
     _assert_pools(dev, ref, f"append nibble dt={dt} D={D} n={n}")
+
+
+@pytest.mark.parametrize("dt", [orc.Q8_0, orc.Q4_0, orc.Q4_1, orc.Q5_0, orc.Q5_1])
+@pytest.mark.parametrize("D,shift", [(32, 0), (32, 2), (96, 4), (128, 8), (256, 6)])
+def test_gather_records_at_any_alignment(dt, D, shift):
+    """Packed records through the 64-record stage: rows of 1, 3, 4 and 8
+    groups, runs that start on 2-, 4- and 16-byte boundaries, sequences that
+    end inside a wave; nothing around them is written.  A block id outside the
+    pool is latched and leaves exactly its records as they were."""
+    import torch
+    from infer_train_amd import InvalidInput
+
+    hkv, nb, bs = 3, 64, 16
+    ctx = np.array([21, 0, 200, 65], np.int32)
+    start = np.array([0, 0, 7, 64], np.int32)
+    tables = random_tables(15, ctx, bs, nb, 16)
+    dev, ref = _pair(nb, bs, hkv, D, dt)
+    seqs = np.repeat(np.arange(4), ctx)
+    pos = np.concatenate([np.arange(c) for c in ctx])
+    slots = slots_for(tables, seqs, pos, bs)
+    k, v = _src(33, len(slots), hkv, D, dt)
+    ref.append(k, v, slots)
+    dev.append(_dev_src(k, dt), _dev_src(v, dt), to_dev(slots))
+    n = ctx - start
+    cu = np.concatenate([[0], np.cumsum(n)[:-1]]).astype(np.int64)
+    rk, rv = ref.gather(tables, ctx, start, cu, int(n.sum()))
+    row = D // 32 * orc.RECORD_BYTES[dt]
+    for bad in (False, True):
+        t = tables.copy()
+        hole = np.zeros(rk.size, bool)
+        if bad:
+            t[2, 5] = nb  # positions 80 .. 95 of sequence 2
+            for h in range(hkv):
+                at = (int(cu[2]) * hkv + h * int(n[2]) + 80 - 7) * row
+                hole[at:at + 16 * row] = True
+        bufs = [torch.full((rk.size + 64,), 0xEE, dtype=torch.uint8, device="cuda:0") for _ in range(2)]
+        dev.gather(to_dev(t), to_dev(ctx), to_dev(start), to_dev(cu), int(n.max()), *(x[shift:] for x in bufs))
+        if bad:
+            with pytest.raises(InvalidInput):
+                dev.check()
+        else:
+            dev.check()
+        for x, want in zip(bufs, (rk, rv)):
+            got = from_dev(x)
+            np.testing.assert_array_equal(got[:shift], 0xEE)
+            np.testing.assert_array_equal(got[shift + want.size:], 0xEE)
+            np.testing.assert_array_equal(got[shift:shift + want.size], np.where(hole, 0xEE, want))
