@@ -172,35 +172,51 @@ extern "C" int32_t it_paged_decode_partition(int32_t dtype, int32_t head_dim, in
     const int64_t n = int64_t(ctx_lens[b]) - (start_pos ? start_pos[b] : 0);
     if (n > max_n) max_n = n;
   }
-  // Resident slots of one round: four workgroups per compute unit, fewer
-  // where the LDS does not hold four.
-  int best = 0, longest_two = 0;
-  int64_t best_rounds = 0;
-  for (int p = 64; p <= 2048; p += 64) {
-    const int64_t parts = max_n > 0 ? (max_n + p - 1) / p : 1;
-    if (parts > kMaxParts) continue;
-    const size_t smem =
-        decode_smem_bytes(dtype, gc, head_dim, p, (p >> log2_bs) + 2, parts * hc * n_seqs);
-    if (smem > kMaxDecodeLds) continue;
-    const int64_t per_cu = std::min<int64_t>(4, int64_t(kMaxDecodeLds / smem));
-    int64_t units = 0;
-    for (int b = 0; b < n_seqs; ++b) {
-      const int64_t n = int64_t(ctx_lens[b]) - (start_pos ? start_pos[b] : 0);
-      if (n > 0) units += (n + p - 1) / p;
+  // Resident slots of one round: `cap` workgroups of two waves per compute
+  // unit (half of four-wave ones past four), fewer where the LDS does not
+  // hold them.
+  struct Plan {
+    int best = 0, longest = 0;  // fewest rounds; longest that keeps the unit full (two workgroups, past cap 4 every one)
+    int64_t rounds = 0;
+  };
+  auto plan = [&](bool full) {
+    Plan r;
+    for (int p = 64; p <= 2048; p += 64) {
+      const int64_t parts = max_n > 0 ? (max_n + p - 1) / p : 1;
+      if (parts > kMaxParts) continue;
+      const SplitShape sh = split_shape(dtype, head_dim, gc, p, (p >> log2_bs) + 2, parts * hc * n_seqs);
+      const size_t smem = split_lds_bytes(dtype, head_dim, gc, p, (p >> log2_bs) + 2, sh.nw, sh.ring);
+      if (smem > kMaxDecodeLds) continue;
+      const int cap = full ? split_resident(dtype, head_dim, sh.nw) : 4;
+      const int64_t per_cu = std::min<int64_t>(cap, int64_t(kMaxDecodeLds / smem));
+      int64_t units = 0;
+      for (int b = 0; b < n_seqs; ++b) {
+        const int64_t n = int64_t(ctx_lens[b]) - (start_pos ? start_pos[b] : 0);
+        if (n > 0) units += (n + p - 1) / p;
+      }
+      const int64_t rounds = (units * hc + per_cu * n_cu - 1) / (per_cu * n_cu);
+      if (!r.best || rounds < r.rounds) {
+        r.best = p;
+        r.rounds = rounds;
+      }
+      if (per_cu >= (full ? cap : 2)) r.longest = p;
     }
-    const int64_t rounds = (units * hc + per_cu * n_cu - 1) / (per_cu * n_cu);
-    if (!best || rounds < best_rounds) {
-      best = p;
-      best_rounds = rounds;
-    }
-    if (per_cu >= 2) longest_two = p;
+    return r;
+  };
+  Plan r = plan(false);
+  // Where registers hold more workgroups, long partitions run shorter beside
+  // more of them.  Short ones stay: 320 tokens at four per unit 28.3 us, 192
+  // at eight 29.3 (32 sequences of 256 to 4096 tokens, 7 heads over one).
+  if (split_resident(dtype, head_dim, 2) > 4 && r.best > 384) {
+    const Plan f = plan(true);
+    if (f.best && (f.rounds <= 2 || f.longest)) r = f;
   }
-  if (!best) return fail(IT_NOT_IMPLEMENTED, "%s: no partition fits (max context %lld)", who, (long long)max_n);
+  if (!r.best) return fail(IT_NOT_IMPLEMENTED, "%s: no partition fits (max context %lld)", who, (long long)max_n);
   // Beyond two rounds the workgroups stream back to back and the machine
   // stays full whatever the size: then the longest partition that still
-  // keeps two workgroups per CU writes the fewest partials and starts the
-  // fewest workgroups.
-  *partition = (best_rounds > 2 && longest_two) ? longest_two : best;
+  // keeps the compute units full (two workgroups each; see above) writes the
+  // fewest partials and starts the fewest workgroups.
+  *partition = (r.rounds > 2 && r.longest) ? r.longest : r.best;
   return IT_OK;
 }
 

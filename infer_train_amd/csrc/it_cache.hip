@@ -369,7 +369,7 @@ __global__ __launch_bounds__(kThreads) void kv_gather_vec(
 // blockIdx.x holds (KV head, 256 groups); blockIdx.y is the sequence.
 // Bound by memory: 4 sequences of 4096 to 16384 tokens, 4 x 256, Q8_0 (194
 // MB): 41.0 us, 4.7 TB/s (2-byte stores straight to the records: 46.9 us);
-// small gathers wait for the stage (1.4 MB of 8 sequences: 3.3 us against 2.9).
+// small gathers wait for the stage (1.4 MB of 16 sequences: 3.3 us against 2.9).
 template <int DT>
 struct GatherRec {
   static constexpr int kBytes = NibFmt<DT>::kRecord;

@@ -138,7 +138,8 @@ inline int split_slot_bytes(int32_t dt, int d) {
 // fp32 reuses the rings.
 inline size_t split_lds_bytes(int32_t dt, int d, int gc, int partition, int max_pages, int nw, int ring) {
   const size_t rings = size_t(nw) * ring * split_slot_bytes(dt, d);
-  const size_t red = size_t(nw) * 8 * d * 4;
+  // Of GC heads; head_dim 256 keeps room for 8 (its partitions were tuned so).
+  const size_t red = size_t(nw) * (d == 128 ? gc : 8) * d * 4;
   const size_t scratch = (dt == IT_BF16 || dt == IT_F16) ? 256 : 512;
   return (rings > red ? rings : red) + size_t(gc) * (partition + 16) * 4 + 2 * size_t(nw) * 8 * 4 + nw * scratch +
          size_t(max_pages + 1) * 4;
@@ -165,6 +166,16 @@ inline SplitShape split_shape(int32_t dt, int d, int gc, int partition, int max_
     if (split_lds_bytes(dt, d, gc, partition, max_pages, 4, r) <= kCu) return {4, r};
   return {4, 2};
 }
+
+// Workgroups of a launch shape that run on one CU, as far as registers go
+// (LDS may hold fewer).  The quantised formats at head_dim 128 take 113-116
+// VGPRs: four waves per SIMD.  Their items are short (16 tokens: 64 bytes a
+// row) and each is a chain of waits, conversions and MFMAs, so four waves
+// hide what two do not; more ring slots did not (Q4_0, 16 sequences of 2048 to
+// 16384 tokens, 8 KV heads: 640-token partitions, eight workgroups per CU,
+// 65 us; 1344 tokens, four, 97 us; three or four slots 67-100 us).  The other
+// kernels: four workgroups (more were slower for the 16-bit formats).
+inline int split_resident(int32_t dt, int d, int nw) { return is_quant(dt) && d == 128 ? 16 / nw : 4; }
 
 // Compile-time loop: f(integral_constant<int, I>) for I in [B, E).
 template <int B, int E>
@@ -460,7 +471,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_split(DecodeArgs a) {
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr size_t kRingAll = size_t(NW) * R * SLOT;
-  constexpr size_t kRed = size_t(NW) * 8 * D * 4;
+  constexpr size_t kRed = size_t(NW) * (D == 128 ? GC : 8) * D * 4;
   char* const ring = smem;
   float* const sc = reinterpret_cast<float*>(smem + (kRingAll > kRed ? kRingAll : kRed));
   const int SP = a.partition + 16;  // plane stride (staggers heads over the banks)

@@ -132,3 +132,28 @@ def test_python_error_mapping():
     p = BlockPool(2)
     with pytest.raises(InvalidInput):
         p.free(1)
+
+
+def test_decode_partition_planner_quantised_128():
+    """Quantised caches at head_dim 128 run up to eight two-wave workgroups
+    per compute unit (LDS permitting): partitions above 384 tokens are planned
+    for that; shorter ones, and every other kernel, for four."""
+    from infer_train_amd import _lib as L
+    from infer_train_amd.kv import decode_partition
+
+    def plan(ctx, hq, hkv, dt, D=128):
+        return decode_partition(dt, D, 16, hq, hkv, ctx, None, 256)
+
+    even = np.full(16, 9216)
+    units = lambda p: int(sum((c + p - 1) // p for c in even)) * 8  # noqa: E731
+    p = plan(even, 32, 8, L.Q4_0)
+    assert p == 576 and units(p) <= 8 * 256 < units(p - 64)  # one round of eight per unit
+    assert plan(even, 32, 8, L.Q8_0) == 576 and plan(even, 32, 8, L.Q5_1) == 576
+    assert plan(even, 32, 8, L.BF16) == plan(even, 32, 8, L.F16)  # four per unit
+    assert plan(even, 32, 8, L.BF16) != 576
+    # 32 x 1024 over 4 KV heads: 128-token partitions at four per unit, kept.
+    assert plan(np.full(32, 1024), 28, 4, L.Q4_0) == 128
+    # Many rounds at any size: the longest partition that leaves room for eight.
+    long = plan(np.full(16, 65536), 32, 8, L.Q4_0)
+    assert 640 <= long <= 1024
+    assert plan(np.full(16, 65536), 64, 8, L.Q4_0) < long  # 8 heads' scores take more LDS
