@@ -176,6 +176,21 @@ def _load() -> C.CDLL:
 lib = _load()
 
 
+def _load_call():
+    """The compiled bindings of the per-step entry points (csrc/it_pycall.cpp):
+    the same functions as `lib`'s, without ctypes' per-argument cost."""
+    try:
+        from . import _call
+    except ImportError as e:
+        raise ImportError(f"{_HERE}/_call.so is missing or does not load ({e}): build it with "
+                          "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+    _call.bind(LIB_PATH)
+    return _call
+
+
+call = _load_call()
+
+
 def check(rc: int) -> None:
     """Raise the OpError subclass for a non-OK status."""
     if rc != OK:

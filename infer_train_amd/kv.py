@@ -10,9 +10,10 @@ import ctypes as C
 import math
 from typing import Optional, Tuple
 
+import numpy as np
 import torch
 
-from ._lib import BF16, CacheDesc, F16, F32, Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, check, lib
+from ._lib import BF16, CacheDesc, F16, F32, Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, call, check, lib
 
 __all__ = ["PagedKvCache", "RopeTable", "flash_attention", "torch_dtype_id", "stream_handle"]
 
@@ -31,6 +32,12 @@ def stream_handle(device: Optional[torch.device] = None) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+# The current stream's handle of a device index, without building a Stream
+# object (1.5 us of each call).
+_raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") else (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     if t is None:
         return None
@@ -41,6 +48,14 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return t.data_ptr()
 
 
+def _check(rc: int) -> None:
+    if rc:
+        check(rc)
+
+
+_DECODE = {"both": call.it_paged_decode, "split": call.it_paged_decode_split, "combine": call.it_paged_decode_combine}
+
+
 class RopeTable:
     """cos/sin of rope_f32's angles (src/backend/arm/rope.rs:30-34) for
     positions [0, max_pos), built on the host in float32 and held on the
@@ -49,7 +64,7 @@ class RopeTable:
     def __init__(self, n_dims: int, max_pos: int, freq_base: float = 10000.0, device: int = 0):
         h = C.c_void_p()
         check(lib.it_rope_table_new(device, n_dims, C.c_float(freq_base), max_pos, C.byref(h)))
-        self._h = h
+        self._h, self._at = h, h.value
         self.n_dims, self.max_pos, self.freq_base, self.device = n_dims, max_pos, freq_base, device
         self._destroy = lib.it_rope_table_destroy
 
@@ -86,6 +101,8 @@ class PagedKvCache:
         check(lib.it_kv_cache_wrap_layers(device, n_layers, self.k_pool.data_ptr(), self.v_pool.data_ptr(),
                                           num_blocks, block_size, n_kv_heads, head_dim, dtype, C.byref(h)))
         self._h = h
+        self._at = h.value  # the handle as the compiled bindings take it
+        self._index = device
         # Bound now: at interpreter exit the module global may already be gone.
         self._destroy = lib.it_kv_cache_destroy
         self.num_blocks, self.block_size, self.n_kv_heads, self.head_dim = num_blocks, block_size, n_kv_heads, head_dim
@@ -109,6 +126,8 @@ class PagedKvCache:
         view.k_pool = self.k_pool[index * lb:(index + 1) * lb]
         view.v_pool = self.v_pool[index * lb:(index + 1) * lb]
         view._h = h
+        view._at = h.value
+        view._index = self._index
         view._destroy = lib.it_kv_cache_destroy
         for name in ("num_blocks", "block_size", "n_kv_heads", "head_dim", "dtype", "page_bytes", "device"):
             setattr(view, name, getattr(self, name))
@@ -183,8 +202,8 @@ class PagedKvCache:
         if slot_mapping.dtype != torch.int64:
             raise TypeError("slot_mapping must be int64")
         n = slot_mapping.numel()
-        check(lib.it_kv_append(self._h, _ptr(k), _ptr(v), torch_dtype_id(k.dtype), _ptr(slot_mapping), n,
-                               stream_handle(self.device)))
+        _check(call.it_kv_append(self._at, _ptr(k), _ptr(v), torch_dtype_id(k.dtype), _ptr(slot_mapping), n,
+                                 _raw_stream(self._index)))
 
     def append_rope(self, rope: RopeTable, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                     slot_mapping: torch.Tensor, positions: torch.Tensor, q_out: Optional[torch.Tensor] = None,
@@ -198,31 +217,31 @@ class PagedKvCache:
             raise TypeError("q, k, v must be float32")
         if q_out is None:
             q_out = torch.empty(q.shape, dtype=q_out_dtype or torch.float32, device=q.device)
-        check(lib.it_kv_append_rope(self._h, rope._h, _ptr(q), q.shape[1], _ptr(k), _ptr(v), _ptr(slot_mapping),
-                                    _ptr(positions), slot_mapping.numel(), _ptr(q_out),
-                                    torch_dtype_id(q_out.dtype), stream_handle(self.device)))
+        _check(call.it_kv_append_rope(self._at, rope._at, _ptr(q), q.shape[1], _ptr(k), _ptr(v), _ptr(slot_mapping),
+                                      _ptr(positions), slot_mapping.numel(), _ptr(q_out),
+                                      torch_dtype_id(q_out.dtype), _raw_stream(self._index)))
         return q_out
 
     def gather(self, block_tables: torch.Tensor, ctx_lens: torch.Tensor, start_pos: Optional[torch.Tensor],
                cu_out: torch.Tensor, max_tokens: int, k_out: torch.Tensor, v_out: torch.Tensor) -> None:
-        check(lib.it_kv_gather(self._h, _ptr(block_tables), block_tables.shape[1], _ptr(ctx_lens), _ptr(start_pos),
-                               _ptr(cu_out), ctx_lens.numel(), max_tokens, _ptr(k_out), _ptr(v_out),
-                               stream_handle(self.device)))
+        _check(call.it_kv_gather(self._at, _ptr(block_tables), block_tables.shape[1], _ptr(ctx_lens), _ptr(start_pos),
+                                 _ptr(cu_out), ctx_lens.numel(), max_tokens, _ptr(k_out), _ptr(v_out),
+                                 _raw_stream(self._index)))
 
     def evict(self, blocks: torch.Tensor) -> None:
-        check(lib.it_kv_evict(self._h, _ptr(blocks), blocks.numel(), stream_handle(self.device)))
+        _check(call.it_kv_evict(self._at, _ptr(blocks), blocks.numel(), _raw_stream(self._index)))
 
     def sync_tables(self, tables: torch.Tensor, seq: torch.Tensor, pos: torch.Tensor, slots: torch.Tensor) -> None:
         """tables[seq[i], pos[i] // bs] = slots[i] // bs (device int32 table [n_seqs, max_blocks])."""
-        check(lib.it_kv_sync_tables(self._h, _ptr(tables), tables.shape[1], tables.shape[0], _ptr(seq), _ptr(pos),
-                                    _ptr(slots), slots.numel(), stream_handle(self.device)))
+        _check(call.it_kv_sync_tables(self._at, _ptr(tables), tables.shape[1], tables.shape[0], _ptr(seq), _ptr(pos),
+                                      _ptr(slots), slots.numel(), _raw_stream(self._index)))
 
     def copy_blocks(self, src: torch.Tensor, dst: torch.Tensor) -> None:
-        check(lib.it_kv_copy_blocks(self._h, _ptr(src), _ptr(dst), src.numel(), stream_handle(self.device)))
+        _check(call.it_kv_copy_blocks(self._at, _ptr(src), _ptr(dst), src.numel(), _raw_stream(self._index)))
 
     # ---- attention --------------------------------------------------------
     def decode_workspace(self, n_seqs: int, n_heads: int, max_tokens: int, partition: int = 512) -> torch.Tensor:
-        nbytes = lib.it_paged_decode_workspace(n_seqs, n_heads, self.head_dim, max_tokens, partition)
+        nbytes = call.it_paged_decode_workspace(n_seqs, n_heads, self.head_dim, max_tokens, partition)
         return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
 
     def decode_partition(self, n_heads: int, ctx_lens, start_pos=None, n_cu: int = 0) -> int:
@@ -241,15 +260,12 @@ class PagedKvCache:
         if scale is None:
             scale = 1.0 / math.sqrt(D)
         if out is None:
-            out = torch.empty(q.shape, dtype=out_dtype or q.dtype, device=q.device)
+            out = torch.empty_like(q, dtype=out_dtype)
         if ws is None:
             ws = self.decode_workspace(n_seqs, n_heads, max_tokens, partition)
-        fn = {"both": lib.it_paged_decode, "split": lib.it_paged_decode_split,
-              "combine": lib.it_paged_decode_combine}[phase]
-        check(fn(self._h, _ptr(q), torch_dtype_id(q.dtype), n_heads, _ptr(block_tables),
-                                  block_tables.shape[1], _ptr(ctx_lens), _ptr(start_pos), n_seqs, max_tokens,
-                                  C.c_float(scale), partition, _ptr(ws), ws.numel(), _ptr(out),
-                                  torch_dtype_id(out.dtype), stream_handle(self.device)))
+        _check(_DECODE[phase](self._at, _ptr(q), torch_dtype_id(q.dtype), n_heads, _ptr(block_tables),
+                              block_tables.shape[1], _ptr(ctx_lens), _ptr(start_pos), n_seqs, max_tokens, scale, partition,
+                              _ptr(ws), ws.numel(), _ptr(out), torch_dtype_id(out.dtype), _raw_stream(self._index)))
         return out
 
     def prefill(self, q: torch.Tensor, cu_q: torch.Tensor, max_q_len: int, block_tables: torch.Tensor,
@@ -262,12 +278,12 @@ class PagedKvCache:
         if out is None:
             out = torch.empty(q.shape, dtype=out_dtype or q.dtype, device=q.device)
         n_seqs, max_blocks = ctx_lens.numel(), block_tables.shape[1]
-        need = lib.it_paged_prefill_workspace(n_heads, self.n_kv_heads, n_seqs, max_q_len, max_blocks, self.block_size)
+        need = call.it_paged_prefill_workspace(n_heads, self.n_kv_heads, n_seqs, max_q_len, max_blocks, self.block_size)
         ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
-        check(lib.it_paged_prefill_ws(self._h, _ptr(q), torch_dtype_id(q.dtype), n_heads, _ptr(cu_q), max_q_len,
-                                      _ptr(block_tables), max_blocks, _ptr(ctx_lens), n_seqs, C.c_float(scale),
+        _check(call.it_paged_prefill_ws(self._at, _ptr(q), torch_dtype_id(q.dtype), n_heads, _ptr(cu_q), max_q_len,
+                                      _ptr(block_tables), max_blocks, _ptr(ctx_lens), n_seqs, scale,
                                       int(bool(causal)), _ptr(ws), need, _ptr(out), torch_dtype_id(out.dtype),
-                                      stream_handle(self.device)))
+                                      _raw_stream(self._index)))
         return out
 
     def __del__(self):
@@ -284,15 +300,12 @@ def decode_partition(dtype: int, head_dim: int, block_size: int, n_heads: int, n
     (it_paged_decode_partition): the smallest multiple of 64 whose non-empty
     units run in the fewest rounds of resident workgroups.  n_cu 0 asks the
     current device."""
-    import numpy as np
-
-    ctx = np.ascontiguousarray(np.asarray(ctx_lens, dtype=np.int32))
-    st = None if start_pos is None else np.ascontiguousarray(np.asarray(start_pos, dtype=np.int32))
+    ctx = np.ascontiguousarray(ctx_lens, dtype=np.int32)
+    st = None if start_pos is None else np.ascontiguousarray(start_pos, dtype=np.int32)
     if st is not None and st.shape != ctx.shape:
         raise ValueError("start_pos must match ctx_lens")
     out = C.c_int32()
-    check(lib.it_paged_decode_partition(dtype, head_dim, block_size, n_heads, n_kv_heads, ctx.ctypes.data,
-                                        None if st is None else st.ctypes.data, ctx.size, n_cu, C.byref(out)))
+    _check(call.it_paged_decode_partition(dtype, head_dim, block_size, n_heads, n_kv_heads, ctx, st, ctx.size, n_cu, out))
     return out.value
 
 
@@ -304,7 +317,7 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Opt
     n_kv = k.shape[0]
     if out is None:
         out = torch.empty_like(q)
-    ws = torch.empty(lib.it_flash_attention_workspace(n_heads, D, n_kv), dtype=torch.uint8, device=q.device)
-    check(lib.it_flash_attention(_ptr(q), _ptr(k), _ptr(v), _ptr(mask), _ptr(out), n_heads, D, n_kv, _ptr(ws),
-                                 ws.numel(), stream_handle(q.device)))
+    ws = torch.empty(call.it_flash_attention_workspace(n_heads, D, n_kv), dtype=torch.uint8, device=q.device)
+    _check(call.it_flash_attention(_ptr(q), _ptr(k), _ptr(v), _ptr(mask), _ptr(out), n_heads, D, n_kv, _ptr(ws),
+                                 ws.numel(), _raw_stream(q.device.index)))
     return out

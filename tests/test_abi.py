@@ -157,3 +157,29 @@ def test_decode_partition_planner_quantised_128():
     long = plan(np.full(16, 65536), 32, 8, L.Q4_0)
     assert 640 <= long <= 1024
     assert plan(np.full(16, 65536), 64, 8, L.Q4_0) < long  # 8 heads' scores take more LDS
+
+
+def test_compiled_bindings_agree_with_ctypes():
+    """infer_train_amd._call passes the same arguments as the ctypes table:
+    same results and statuses (nothing here reaches a device), and what ctypes
+    refuses stays refused."""
+    from infer_train_amd import _lib as L
+
+    for args in ((32, 28, 128, 4097, 512), (1, 1, 128, 0, 64), (0, 1, 128, 5, 64), (65535, 64, 256, 2 ** 31 - 1, 64)):
+        assert L.call.it_paged_decode_workspace(*args) == L.lib.it_paged_decode_workspace(*args)
+    assert L.call.it_paged_prefill_workspace(32, 8, 1, 500, 1032, 16) == L.lib.it_paged_prefill_workspace(32, 8, 1, 500, 1032, 16) > 0
+    assert L.call.it_paged_prefill_workspace(32, 8, 8, 512, 160, 16) == 0  # 512 workgroups without cuts
+    ctx, out = np.array([1024, 4096, 17], np.int32), C.c_int32()
+    assert L.call.it_paged_decode_partition(L.BF16, 128, 16, 28, 4, ctx, None, 3, 256, out) == L.OK
+    want = C.c_int32()
+    assert L.lib.it_paged_decode_partition(L.BF16, 128, 16, 28, 4, ctx.ctypes.data, None, 3, 256, C.byref(want)) == L.OK
+    assert out.value == want.value > 0
+    assert L.call.it_kv_append(None, None, None, L.BF16, None, 1, None) == L.INVALID_INPUT
+    assert b"NULL" in L.lib.it_last_error()
+    assert L.call.it_paged_prefill_ws(None, None, L.BF16, 8, None, 1, None, 1, None, 1, 0.1, 1, None, 0, None, L.BF16,
+                                      None) == L.INVALID_INPUT
+    with pytest.raises(TypeError):
+        L.call.it_kv_evict(None, None, 0)
+    for bad in ((None, None, 1.0, None), (1.5, None, 0, None), (None, "x", 0, None)):
+        with pytest.raises(C.ArgumentError):
+            L.call.it_kv_evict(*bad)
