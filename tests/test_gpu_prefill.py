@@ -208,6 +208,27 @@ def test_prefill_unit_order_ragged(n_seqs, hq, hkv, causal):
     assert_close(from_dev(out), want, RTOL, ATOL, what=f"prefill order n_seqs={n_seqs}")
 
 
+@pytest.mark.parametrize("n_seqs,hq,hkv,equal,causal", [
+    (16, 32, 4, False, True),   # 256 workgroups: one per CU, ids in pair order
+    (22, 24, 3, False, True),   # 264: searched 64 block counts at a time
+    (24, 24, 3, False, False), (25, 24, 3, False, True), (64, 14, 2, False, True),
+    (24, 24, 3, True, True),    # equal sequences: the rank's unit by division
+])
+def test_prefill_unit_order_past_one_round(n_seqs, hq, hkv, equal, causal):
+    """Grids of more than 256 workgroups take the longest-first order, smaller
+    ones do not: both sides of the line and of the order's own branches.  Every
+    row against the oracle."""
+    rng = np.random.RandomState(700 + n_seqs)
+    q_lens = np.full(n_seqs, 97) if equal else rng.choice([0, 1, 31, 32, 33, 65, 100], n_seqs)
+    q_lens[0] = 97
+    ctx = q_lens + (63 if equal else rng.choice([0, 1, 63, 64, 200], n_seqs))
+    assert (4 * n_seqs * hkv > 256) == (n_seqs != 16)  # four query blocks of 32 rows (hq / hkv of 7 or 8)
+    dev, ref, tables, ctx, cu, q, td = _setup(orc.BF16, hq, hkv, ctx, q_lens, seed=700 + n_seqs)
+    out, scale = _run(dev, tables, ctx, cu, q, td, hq, causal=causal)
+    want = ref.prefill(widen(q, orc.BF16), hq, cu, tables, ctx, scale, causal=causal)
+    assert_close(from_dev(out), want, RTOL, ATOL, what=f"prefill order n_seqs={n_seqs} equal={equal}")
+
+
 @pytest.mark.parametrize("dt,hq,hkv,ctx,q_lens,causal", [
     (orc.BF16, 8, 2, [2100], [70], True),          # one long context, few rows: 8 cuts
     (orc.F16, 7, 1, [4096, 130], [33, 1], True),   # 7 waves; a unit too short to cut beside long ones
