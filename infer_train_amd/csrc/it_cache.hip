@@ -164,8 +164,8 @@ __global__ __launch_bounds__(kThreads) void kv_append_quant(
 //    all: each such instruction touches 64 scattered pieces.)
 //  - Quantise in that layout: eight lanes per 32-group (quant_group).
 //  - The wave's 1024 int8 and 32 fp16 scales go through a wave-private
-//    1088-byte LDS stage (same-wave LDS operations stay in order), and lane
-//    L stores bytes 16 L .. 16 L + 15 of the group's int8, one 16-byte
+//    1088-byte LDS stage (wave_lds_fence keeps the order), and lane L
+//    stores bytes 16 L .. 16 L + 15 of the group's int8, one 16-byte
 //    vector (a 1 KiB store instruction); the first lane of each row stores
 //    the row's D / 32 scales as one 4-, 8- or 16-byte word.
 // blockIdx.y selects K (0) or V (1).
@@ -208,12 +208,19 @@ __global__ __launch_bounds__(kThreads) void kv_append_q8_wide(
       *reinterpret_cast<uint32_t*>(st + 256 * j + 4 * lane) = q.qs;
       if ((lane & 7) == 0) *reinterpret_cast<uint16_t*>(st + 1024 + 2 * (8 * j + (lane >> 3))) = uint16_t(q.meta);
     }
-    const uint4 w = *reinterpret_cast<const uint4*>(st + 16 * lane);
+    wave_lds_fence();
+    const uint4 w = lds_read<uint4>(st + 16 * lane);
     uint4 sw = make_uint4(0u, 0u, 0u, 0u);
     const char* const ss = st + 1024 + srow * (D / 16);  // the row's D / 32 scales
-    if constexpr (LPR == 16) sw = *reinterpret_cast<const uint4*>(ss);
-    else if constexpr (LPR == 8) sw.x = reinterpret_cast<const uint2*>(ss)->x, sw.y = reinterpret_cast<const uint2*>(ss)->y;
-    else sw.x = *reinterpret_cast<const uint32_t*>(ss);
+    if constexpr (LPR == 16) {
+      sw = lds_read<uint4>(ss);
+    } else if constexpr (LPR == 8) {
+      const uint2 s2 = lds_read<uint2>(ss);
+      sw.x = s2.x, sw.y = s2.y;
+    } else {
+      sw.x = lds_read<uint32_t>(ss);
+    }
+    wave_lds_fence();  // the next group's stores follow
     if (row < n_rows && sl >= 0) {
       const int h = log2_hkv >= 0 ? row & (hkv - 1) : row % hkv;
       if (sl >= n_slots) {
@@ -239,7 +246,7 @@ __global__ __launch_bounds__(kThreads) void kv_append_q8_wide(
 //  - Loads: eight instructions of 1 KiB, all issued before the first is used.
 //  - Quantise: eight lanes per 32-group (quant_group).
 //  - The groups' nibble bytes and words go through a wave-private LDS stage
-//    (same-wave LDS operations stay in order); lane L then stores group L: its
+//    (wave_lds_fence keeps the order); lane L then stores group L: its
 //    16 nibble bytes as one vector, its qh word, its d or (d, m).
 // Bound by memory and, near it, by the quantiser's VALU.  4096 tokens of 4 x
 // 256, Q4_0 (38 MB): 8.5 us, 4.5 TB/s (one vector per lane, 4- and 2-byte
@@ -283,10 +290,12 @@ __global__ __launch_bounds__(kThreads) void kv_append_nib_wide(
         if constexpr (N::kQ5) st_h[wave][g] = q.qh;
       }
     }
-    const uint4 w = *reinterpret_cast<const uint4*>(&st_q[wave][4 * lane]);
+    wave_lds_fence();
+    const uint4 w = lds_read<uint4>(&st_q[wave][4 * lane]);
     const uint32_t meta = st_m[wave][lane];
     uint32_t qh = 0u;
     if constexpr (N::kQ5) qh = st_h[wave][lane];
+    wave_lds_fence();  // the next chunk's stores follow
     if (row < n_rows && sl >= 0) {
       const int g = lane % NG;
       const int h = row - tok * hkv;
@@ -363,8 +372,8 @@ __global__ __launch_bounds__(kThreads) void kv_gather_vec(
 // types.rs:24-32), ggml's block_q5_0 {u16 d; u8 qh[4]; qs} (22) and block_q5_1
 // {u16 d; u16 m; u8 qh[4]; qs} (24).  A sequence's records of one KV head
 // follow one another, so a wave's 64 are one run of a multiple of 128 bytes:
-// they are packed in a wave-private LDS stage (same-wave LDS operations stay
-// in order) and stored as 16-byte vectors, or 4- or 2-byte ones where the run
+// they are packed in a wave-private LDS stage (wave_lds_fence keeps the
+// order) and stored as 16-byte vectors, or 4- or 2-byte ones where the run
 // starts unaligned (groups of a row that is not a multiple of 8 records).
 // blockIdx.x holds (KV head, 256 groups); blockIdx.y is the sequence.
 // Bound by memory: 4 sequences of 4096 to 16384 tokens, 4 x 256, Q8_0 (194
@@ -470,6 +479,7 @@ __global__ __launch_bounds__(kThreads) void kv_gather_quant(
       put(q[w][c].w);
     }
   }
+  wave_lds_fence();
   const char* const sk = stage[threadIdx.x >> 6][0];
   const char* const sv = stage[threadIdx.x >> 6][1];
   char* const ok = kout + rec0;
@@ -483,8 +493,8 @@ __global__ __launch_bounds__(kThreads) void kv_gather_quant(
 #pragma unroll
     for (int c = 0; c < kPieces; ++c) {
       const int p = min(lane + 64 * c, 64 * REC / int(sizeof(U)) - 1);
-      xk[c] = reinterpret_cast<const U*>(sk)[p];
-      xv[c] = reinterpret_cast<const U*>(sv)[p];
+      xk[c] = lds_read<U>(sk + p * sizeof(U));
+      xv[c] = lds_read<U>(sv + p * sizeof(U));
     }
 #pragma unroll
     for (int c = 0; c < kPieces; ++c) {

@@ -106,6 +106,23 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
   return v;
 }
 
+// Between a wave's stores to an LDS stage and other lanes' loads of it, and
+// before the stage is written again.  The hardware keeps one wave's LDS
+// operations in order; this keeps the compiler from moving them past each
+// other (a lane's own stores and loads need not overlap, and types may differ).
+// No instruction is emitted.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// A U of an LDS stage that was written through other types (aligned to U).
+template <class U>
+__device__ __forceinline__ U lds_read(const void* p) {
+  U x;
+  __builtin_memcpy(&x, __builtin_assume_aligned(p, sizeof(U)), sizeof(U));
+  return x;
+}
+
 // Load helpers: 16-byte vector loads/stores on raw byte addresses.
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ __forceinline__ void st16(void* p, uint4 v) { *reinterpret_cast<uint4*>(p) = v; }
