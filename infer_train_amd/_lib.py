@@ -178,13 +178,14 @@ lib = _load()
 
 def _load_call():
     """The compiled bindings of the per-step entry points (csrc/it_pycall.cpp):
-    the same functions as `lib`'s, without ctypes' per-argument cost."""
+    the same functions as `lib`'s, without ctypes' per-argument cost.  A call
+    with an argument other than an int, a float or None goes through `lib`."""
     try:
         from . import _call
     except ImportError as e:
         raise ImportError(f"{_HERE}/_call.so is missing or does not load ({e}): build it with "
                           "`python -c 'import __graft_entry__ as g; g.build()'`") from e
-    _call.bind(LIB_PATH)
+    _call.bind(LIB_PATH, lib)
     return _call
 
 

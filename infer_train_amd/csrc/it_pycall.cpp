@@ -4,13 +4,17 @@
 // ctypes converts each argument through Python-level descriptors: an 18-
 // argument call costs ~3 us before the library sees it, more than a kernel
 // launch.  Here the C signature of each function (include/it_kv.h) drives the
-// conversion at compile time.  Arguments are what the ctypes table takes:
-// integers (masked to the parameter's width), addresses, None or host buffers
-// for pointers, and floats; the result is the function's integer.  The GIL is released
-// around the call, as ctypes does.
+// conversion at compile time, for the arguments a call nearly always has: ints
+// (masked to the parameter's width), ints or None for pointers, floats or ints
+// for floats.  A call with any other argument is handed to the ctypes function
+// as it is, so what ctypes takes (__index__, ctypes instances, _as_parameter_)
+// is taken and what it refuses is refused with its error (and a str, which
+// c_void_p would take for the address of its characters).  Only
+// it_paged_decode_partition takes more: its arrays are host memory and may be
+// given as buffers.  The GIL is released around the call, as ctypes does.
 //
 // The functions are looked up in the library that the package has loaded
-// (bind(path)), not linked.
+// (bind(path, lib)), not linked.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -23,79 +27,97 @@
 #include "it_kv.h"
 
 namespace {
-PyObject* argument_error = nullptr;  // ctypes.ArgumentError: what the ctypes table raises
+PyObject* argument_error = nullptr;  // ctypes.ArgumentError
 
-// An int for an integer; an int, None or an object with a contiguous buffer
-// for a pointer; a number for a float.  Anything else is refused.
-template <class T>
-T convert(PyObject* o) {
+// The value of an argument that needs no more than this; false: ctypes decides.
+// kHost: the function's pointers are host memory, given as addresses or as
+// buffers (const: of one dimension or more; else writable).
+template <bool kHost, class T>
+bool convert(PyObject* o, T& v) {
   if constexpr (std::is_floating_point_v<T>) {
-    return static_cast<T>(PyFloat_AsDouble(o));
+    if (!PyFloat_Check(o) && !PyLong_Check(o)) return false;
+    const double d = PyFloat_AsDouble(o);  // an int past the double range fails
+    if (d == -1.0 && PyErr_Occurred()) {
+      PyErr_Clear();
+      return false;
+    }
+    v = static_cast<T>(d);
   } else if (PyLong_Check(o)) {
-    if constexpr (std::is_pointer_v<T>) return reinterpret_cast<T>(PyLong_AsVoidPtr(o));
-    else return static_cast<T>(PyLong_AsUnsignedLongLongMask(o));
-  } else if (std::is_pointer_v<T> && o == Py_None) {
-    return T{};
-  } else if (std::is_pointer_v<T> && PyObject_CheckBuffer(o)) {
-    // Host memory (a numpy array, a ctypes value); the caller keeps it.
+    const unsigned long long x = PyLong_AsUnsignedLongLongMask(o);
+    if constexpr (std::is_pointer_v<T>) v = reinterpret_cast<T>(static_cast<uintptr_t>(x));
+    else v = static_cast<T>(x);
+  } else if constexpr (std::is_pointer_v<T>) {
+    v = T{};
+    if (o == Py_None) return true;
+    if (!kHost || !PyObject_CheckBuffer(o)) return false;
+    constexpr bool kConst = std::is_const_v<std::remove_pointer_t<T>>;
     Py_buffer b;
-    if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE)) return T{};
-    void* const p = b.buf;
+    if (PyObject_GetBuffer(o, &b, kConst ? PyBUF_ND : PyBUF_ND | PyBUF_WRITABLE)) {
+      PyErr_Clear();
+      return false;
+    }
+    const bool taken = !kConst || b.ndim > 0;
+    v = reinterpret_cast<T>(b.buf);  // the caller keeps the object for the call
     PyBuffer_Release(&b);
-    if constexpr (std::is_pointer_v<T>) return reinterpret_cast<T>(p);
+    return taken;
   } else {
-    PyErr_Format(argument_error, "int expected instead of %s instance", Py_TYPE(o)->tp_name);
+    return false;
   }
-  return T{};
+  return true;
 }
 
-template <class F>
+template <bool kHost, class F>
 struct Call;
-template <class R, class... A>
-struct Call<R (*)(A...)> {
+template <bool kHost, class R, class... A>
+struct Call<kHost, R (*)(A...)> {
   using Fn = R (*)(A...);
   template <size_t... I>
-  static PyObject* run(Fn f, PyObject* const* args, std::index_sequence<I...>) {
-    std::tuple<A...> v{convert<A>(args[I])...};  // braces: converted in order
-    if (PyErr_Occurred()) return nullptr;
+  static PyObject* run(Fn f, PyObject* ctypes, PyObject* const* args, Py_ssize_t n, std::index_sequence<I...>) {
+    std::tuple<A...> v{};
+    if (n != Py_ssize_t(sizeof...(A)) || !(convert<kHost>(args[I], std::get<I>(v)) && ...)) {
+      for (Py_ssize_t i = 0; i < n; ++i)
+        if (PyUnicode_Check(args[i])) return PyErr_Format(argument_error, "argument %zd: a str is not an address", i + 1);
+      return PyObject_Vectorcall(ctypes, args, size_t(n), nullptr);
+    }
     R r;
     Py_BEGIN_ALLOW_THREADS r = f(std::get<I>(v)...);
     Py_END_ALLOW_THREADS
     if constexpr (std::is_signed_v<R>) return PyLong_FromLongLong(r);
     else return PyLong_FromUnsignedLongLong(r);
   }
-  static PyObject* run(const char* name, Fn f, PyObject* const* args, Py_ssize_t n) {
+  static PyObject* run(const char* name, Fn f, PyObject* ctypes, PyObject* const* args, Py_ssize_t n) {
     if (!f) {
       PyErr_Format(PyExc_RuntimeError, "%s: bind() the library first", name);
       return nullptr;
     }
-    if (n != Py_ssize_t(sizeof...(A))) {
-      PyErr_Format(PyExc_TypeError, "%s takes %zd arguments (%zd given)", name, Py_ssize_t(sizeof...(A)), n);
-      return nullptr;
-    }
-    return run(f, args, std::index_sequence_for<A...>{});
+    return run(f, ctypes, args, n, std::index_sequence_for<A...>{});
   }
 };
 
-#define IT_CALLS(X)                                                                                        \
-  X(it_kv_append) X(it_kv_append_rope) X(it_kv_gather) X(it_kv_evict) X(it_kv_sync_tables)                 \
-  X(it_kv_copy_blocks) X(it_paged_decode_workspace) X(it_paged_decode_partition) X(it_paged_decode)        \
-  X(it_paged_decode_split) X(it_paged_decode_combine) X(it_paged_prefill_workspace) X(it_paged_prefill_ws) \
-  X(it_flash_attention_workspace) X(it_flash_attention)
+#define IT_CALLS(X)                                                                                                      \
+  X(it_kv_append, false) X(it_kv_append_rope, false) X(it_kv_gather, false) X(it_kv_evict, false)                        \
+  X(it_kv_sync_tables, false) X(it_kv_copy_blocks, false) X(it_paged_decode_workspace, false)                            \
+  X(it_paged_decode_partition, true) X(it_paged_decode, false) X(it_paged_decode_split, false)                           \
+  X(it_paged_decode_combine, false) X(it_paged_prefill_workspace, false) X(it_paged_prefill_ws, false)                   \
+  X(it_flash_attention_workspace, false) X(it_flash_attention, false)
 
-#define IT_WRAP(name)                                                               \
+#define IT_WRAP(name, host)                                                         \
   decltype(&name) p_##name = nullptr;                                               \
+  PyObject* c_##name = nullptr;                                                     \
   PyObject* py_##name(PyObject*, PyObject* const* args, Py_ssize_t n) {             \
-    return Call<decltype(&name)>::run(#name, p_##name, args, n);                    \
+    return Call<host, decltype(&name)>::run(#name, p_##name, c_##name, args, n);    \
   }
 IT_CALLS(IT_WRAP)
 
-PyObject* bind(PyObject*, PyObject* arg) {
-  const char* path = PyUnicode_AsUTF8(arg);
-  if (!path) return nullptr;
+PyObject* bind(PyObject*, PyObject* args) {
+  const char* path;
+  PyObject* table;
+  if (!PyArg_ParseTuple(args, "sO", &path, &table)) return nullptr;
   void* lib = dlopen(path, RTLD_NOW | RTLD_NOLOAD);
   if (!lib) return PyErr_Format(PyExc_ImportError, "%s is not loaded", path);
-#define IT_BIND(name)                                                                                             \
+#define IT_BIND(name, host)                                                                                       \
+  Py_XSETREF(c_##name, PyObject_GetAttrString(table, #name));                                                     \
+  if (!c_##name) return nullptr;                                                                                  \
   p_##name = reinterpret_cast<decltype(p_##name)>(dlsym(lib, #name));                                             \
   if (!p_##name) return PyErr_Format(PyExc_ImportError, "%s does not export " #name, path);
   IT_CALLS(IT_BIND)
@@ -103,8 +125,8 @@ PyObject* bind(PyObject*, PyObject* arg) {
 }
 
 PyMethodDef methods[] = {
-    {"bind", bind, METH_O, "Look the entry points up in the loaded library at this path."},
-#define IT_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_##name)), METH_FASTCALL, nullptr},
+    {"bind", bind, METH_VARARGS, "bind(path, lib): the entry points of the loaded library at this path, lib its ctypes table."},
+#define IT_METHOD(name, host) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_##name)), METH_FASTCALL, nullptr},
     IT_CALLS(IT_METHOD){nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_call", "Bindings of include/it_kv.h's per-step entry points.", -1, methods,
                       nullptr, nullptr, nullptr, nullptr};

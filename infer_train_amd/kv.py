@@ -259,6 +259,8 @@ class PagedKvCache:
         n_seqs, n_heads, D = q.shape
         if scale is None:
             scale = 1.0 / math.sqrt(D)
+        elif type(scale) is not float:
+            scale = C.c_float(scale).value
         if out is None:
             out = torch.empty_like(q, dtype=out_dtype)
         if ws is None:
@@ -275,6 +277,8 @@ class PagedKvCache:
         total, n_heads, D = q.shape
         if scale is None:
             scale = 1.0 / math.sqrt(D)
+        elif type(scale) is not float:
+            scale = C.c_float(scale).value
         if out is None:
             out = torch.empty(q.shape, dtype=out_dtype or q.dtype, device=q.device)
         n_seqs, max_blocks = ctx_lens.numel(), block_tables.shape[1]

@@ -183,3 +183,67 @@ def test_compiled_bindings_agree_with_ctypes():
     for bad in ((None, None, 1.0, None), (1.5, None, 0, None), (None, "x", 0, None)):
         with pytest.raises(C.ArgumentError):
             L.call.it_kv_evict(*bad)
+
+
+def test_compiled_bindings_take_and_refuse_what_ctypes_does():
+    """Arguments other than plain ints, floats and None: the compiled binding
+    gives the ctypes table's result or its exception type, argument by
+    argument.  No function here reaches a device: the cache is NULL, or host
+    arithmetic answers."""
+    import torch
+
+    from infer_train_amd import _lib as L
+
+    class Index:
+        def __index__(self):
+            return 4097
+
+    class Parameter:
+        _as_parameter_ = 4097
+
+    def outcome(f, *args):
+        try:
+            return f(*args)
+        except Exception as e:  # noqa: BLE001
+            return type(e)
+
+    arr = np.zeros(4, np.int32)
+    odd = [np.int64(4097), np.int32(4097), np.uint8(7), torch.tensor(4097), Index(), Parameter(), C.c_int32(4097), True,
+           2 ** 40 + 4097, -1, 4097.0, np.float32(3.0), None, arr, arr[:1], b"abcd", bytearray(8), [1], C.byref(C.c_int32())]
+    taken = 0
+    for x in odd:
+        for i in range(5):
+            args = [32, 28, 128, 4097, 512]
+            args[i] = x
+            want = outcome(L.lib.it_paged_decode_workspace, *args)
+            assert outcome(L.call.it_paged_decode_workspace, *args) == want, (x, i)
+            taken += not isinstance(want, type)
+    assert taken >= 5 * 8  # numpy integers, a 0-d tensor, __index__, _as_parameter_, ctypes values, bool, wide and negative ints
+    assert L.call.it_paged_decode_workspace(32, 28, 128, np.int64(4097), 512) == L.lib.it_paged_decode_workspace(32, 28, 128, 4097, 512)
+    # Addresses (None and 0 keep the call from any device): a buffer is not one.
+    for x in odd + [C.c_void_p(), C.c_void_p(64)]:
+        for i in (1, 3):
+            args = [None, None, 0, None]
+            args[i] = x
+            assert outcome(L.call.it_kv_evict, *args) == outcome(L.lib.it_kv_evict, *args), (x, i)
+    for x in (arr, arr[:1], np.int64(64), bytearray(8)):
+        with pytest.raises(C.ArgumentError):
+            L.call.it_kv_append(None, x, None, L.BF16, None, 1, None)
+    for args in ((), (32,), (32, 28, 128, 4097), (32, 28, 128, 4097, 512, 1)):
+        assert outcome(L.call.it_paged_decode_workspace, *args) == outcome(L.lib.it_paged_decode_workspace, *args), args
+    for scale in (1, np.float32(0.5), np.float64(0.5), torch.tensor(0.5), 10 ** 400, "0.5", None):
+        args = [None, None, L.BF16, 8, None, 1, None, 1, None, 1, scale, 1, None, 0, None, L.BF16, None]
+        assert outcome(L.call.it_paged_prefill_ws, *args) == outcome(L.lib.it_paged_prefill_ws, *args), scale
+    # The planner's host arrays: contiguous ones are read, others are not taken.
+    ctx, out = np.array([1024, 4096, 17], np.int32), C.c_int32()
+    planner = [L.BF16, 128, 16, 28, 4, ctx, None, 3, 256, out]
+    assert L.call.it_paged_decode_partition(*planner) == L.OK and out.value > 0
+    for i, x in ((5, np.repeat(ctx, 2)[::2]), (5, np.int64(64)), (9, np.int64(64))):
+        bad = list(planner)
+        bad[i] = x
+        with pytest.raises(C.ArgumentError):
+            L.call.it_paged_decode_partition(*bad)
+    for n in (np.int64(3), torch.tensor(3)):
+        out.value = 0
+        assert L.call.it_paged_decode_partition(*planner[:5], ctx.ctypes.data, None, n, 256, C.addressof(out)) == L.OK
+        assert out.value > 0
