@@ -212,7 +212,8 @@ def test_prefill_unit_order_ragged(n_seqs, hq, hkv, causal):
     (16, 32, 4, False, True),   # 256 workgroups: one per CU, ids in pair order
     (22, 24, 3, False, True),   # 264: searched 64 block counts at a time
     (24, 24, 3, False, False), (25, 24, 3, False, True), (64, 14, 2, False, True),
-    (24, 24, 3, True, True),    # equal sequences: the rank's unit by division
+    (24, 24, 3, True, True),    # equal sequences: pairs dealt to the XCDs in runs
+    (25, 24, 3, True, True),    # 75 pairs: one by one
 ])
 def test_prefill_unit_order_past_one_round(n_seqs, hq, hkv, equal, causal):
     """Grids of more than 256 workgroups take the longest-first order, smaller
