@@ -427,7 +427,10 @@ int32_t it_paged_prefill(const it_kv_cache* cache, const void* q, int32_t q_dtyp
                          int32_t causal, void* out, int32_t out_dtype, void* stream);
 /* Bytes of device workspace with which it_paged_prefill_ws can cut a call's
  * work over the keys; 0 if it would not (a launch of this size fills the
- * device without).  Bounded: at most 70 MB. */
+ * device without).  Bounded: at most 70 MB.  max_blocks x block_size bounds the
+ * contexts: a caller that knows the longest asks with its blocks instead of the
+ * table's width, and passes no workspace where the answer is 0 (then the call
+ * is one launch).  Where a workspace is passed it is of the table's width. */
 size_t it_paged_prefill_workspace(int32_t n_heads, int32_t n_kv_heads, int32_t n_seqs, int32_t max_q_len,
                                   int32_t max_blocks, int32_t block_size);
 /* it_paged_prefill with a workspace (device, 256-byte aligned,
@@ -435,7 +438,11 @@ size_t it_paged_prefill_workspace(int32_t n_heads, int32_t n_kv_heads, int32_t n
  * lengths leave the device with few workgroups (a chunk of one long
  * context), the keys of each query block are divided among several, whose
  * fp32 partial (m, l, O) go through the workspace to a second kernel that
- * merges them. */
+ * merges them.  The number of divisions follows from all sequences of the call
+ * and from max_blocks, so a row's result may differ between batches, and
+ * between calls with and without a workspace, by the rounding of its
+ * probabilities to 16 bits against other maxima; without one it depends on the
+ * row's own sequence alone. */
 int32_t it_paged_prefill_ws(const it_kv_cache* cache, const void* q, int32_t q_dtype, int32_t n_heads,
                             const int32_t* cu_q, int32_t max_q_len, const int32_t* block_tables,
                             int32_t max_blocks, const int32_t* ctx_lens, int32_t n_seqs, float scale,

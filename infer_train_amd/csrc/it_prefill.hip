@@ -98,8 +98,10 @@ struct PrefillArgs {
   int n_heads, n_kv_heads, group, q_tiles, max_blocks, log2_bs, causal, out_f32;
   int n_qb;               // query blocks per (sequence, KV head)
   int n_seqs;
+  int n_wg;               // query blocks of all (sequence, KV head) pairs, by max_q_len
   Divisor place, heads;   // of equal_place: pairs per XCD (or all pairs) and KV heads
   int max_tiles;          // tiles the workspace holds; 0: units are not split
+  int* ws_splits;         // what splits the main kernel found, for the combine
   float4* ws_o;           // [max_tiles][waves][16][64]: a wave's O^T registers, 16 bytes of each lane
   float2* ws_ml;          // [max_tiles][waves][64]: (max, sum) of each lane's query
 };
@@ -271,28 +273,31 @@ __device__ __forceinline__ void equal_unit(const UnitOrder& o, const EqualPlace&
   u.ctx = __builtin_amdgcn_readfirstlane(o.before) + u.q_len;
 }
 
-// The number of units, and of the cuts they take.
-template <bool kCut>
-__device__ __forceinline__ void load_order(const PrefillArgs& a, UnitOrder& o) {
-  const int lane = int(threadIdx.x & 63);
+__device__ __forceinline__ void count_units(const PrefillArgs& a, UnitOrder& o) {
   o.n_units = a.n_kv_heads * wave_total(o.nq);
+}
+// The cuts of a unit, and the number of units where they may be more than one:
+// most calls whose table only may be long are told so by their longest unit.
+__device__ __forceinline__ void price_cuts(const PrefillArgs& a, UnitOrder& o) {
+  const int lane = int(threadIdx.x & 63);
   o.splits = 1;
-  if (kCut && o.n_units > 0 && 2 * o.n_units <= a.max_tiles) {  // uniform
-    // Lane i prices i + 1 cuts, in 16ths of a key block's time.
-    const int most = most_blocks(a, o) - 1;
-    const int work = (o.nq * (key_blocks(first_end(a, o)) + key_blocks(last_end(a, o)))) >> 1;
-    const int S = lane + 1;
-    const int mean16 = int(int64_t(a.n_kv_heads) * wave_total(work) * 16 / o.n_units);
-    const int cut16 = S > 1 ? 16 * kCutCost : 0;
-    const int rounds = (o.n_units * S + kCus - 1) / kCus;
-    int cost = max(rounds * (mean16 / S + cut16), 16 * most / S + cut16);
-    if (S > kMaxCuts || (S > 1 && (o.n_units * S > a.max_tiles || most < kCutMin * S))) cost = INT_MAX;
-    // Only for a gain of a tenth.
-    if (S == 1) cost -= cost / 10;
-    const float c = -float(cost);
-    const float best = group_max<64>(c);
-    o.splits = __builtin_amdgcn_readfirstlane(int(__builtin_ctzll(__builtin_amdgcn_ballot_w64(c == best)))) + 1;
-  }
+  const int most = most_blocks(a, o) - 1;
+  if (most < 2 * kCutMin) return;  // uniform
+  count_units(a, o);
+  if (o.n_units == 0 || 2 * o.n_units > a.max_tiles) return;  // uniform
+  // Lane i prices i + 1 cuts, in 16ths of a key block's time.
+  const int work = (o.nq * (key_blocks(first_end(a, o)) + key_blocks(last_end(a, o)))) >> 1;
+  const int S = lane + 1;
+  const int mean16 = int(int64_t(a.n_kv_heads) * wave_total(work) * 16 / o.n_units);
+  const int cut16 = S > 1 ? 16 * kCutCost : 0;
+  const int rounds = (o.n_units * S + kCus - 1) / kCus;
+  int cost = max(rounds * (mean16 / S + cut16), 16 * most / S + cut16);
+  if (S > kMaxCuts || (S > 1 && (o.n_units * S > a.max_tiles || most < kCutMin * S))) cost = INT_MAX;
+  // Only for a gain of a tenth.
+  if (S == 1) cost -= cost / 10;
+  const float c = -float(cost);
+  const float best = group_max<64>(c);
+  o.splits = __builtin_amdgcn_readfirstlane(int(__builtin_ctzll(__builtin_amdgcn_ballot_w64(c == best)))) + 1;
 }
 
 // The unit of rank r < o.n_units.
@@ -347,6 +352,26 @@ __device__ __forceinline__ void unit_of_rank(const PrefillArgs& a, const UnitOrd
   u.ctx = __builtin_amdgcn_readlane(o.before, idx) + u.q_len;
 }
 
+// The place of this workgroup where the lengths do not matter (more sequences
+// than lanes, or a grid that runs at once): ids are remapped so that all query
+// blocks of one (sequence, KV head), which stream the same K/V pages, run on
+// one XCD and share its L2; an XCD holding ppx whole pairs takes query rank
+// k / ppx of pair k % ppx, its longest causal blocks first.
+__device__ __forceinline__ void pair_place(const PrefillArgs& a, PrefillUnit& u) {
+  const int n_full = a.n_wg & ~7;
+  const int id = blockIdx.x;
+  const int per_xcd = n_full >> 3;
+  int k = id >> 3;
+  if (per_xcd > 0 && per_xcd % a.n_qb == 0) {
+    const int ppx = per_xcd / a.n_qb;
+    k = (k % ppx) * a.n_qb + k / ppx;
+  }
+  const int unit = id < n_full ? (id & 7) * per_xcd + k : id;
+  const int pair = unit / a.n_qb;
+  u.qb = a.n_qb - 1 - (unit - pair * a.n_qb);
+  u.kvh = pair % a.n_kv_heads, u.b = pair / a.n_kv_heads;
+}
+
 // Keys the unit's query block needs: up to its last valid query's position.
 __device__ __forceinline__ int unit_keys(const PrefillArgs& a, int q_len, int ctx, int qb) {
   const int wg_q = kQB * a.q_tiles;
@@ -381,21 +406,38 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   // first ends.  Up to kOrderSeqs sequences: id = rank in the longest-first
   // order (unit_of_rank), so every XCD gets the same share of long and short
   // units whatever the sequences' lengths.
+  // The arguments that place the workgroup, loaded at once (the compiler loads
+  // each where it is used: a round trip after another).
+  asm volatile("" ::"s"(a.cu_q), "s"(a.ctx_lens), "s"(a.n_seqs), "s"(a.n_kv_heads), "s"(a.q_tiles), "s"(a.n_qb), "s"(a.n_wg),
+               "s"(a.causal), "s"(a.group), "s"(a.place.d), "s"(a.place.inv), "s"(a.heads.d), "s"(a.heads.inv));
   PrefillUnit u;
   int cut = 0, splits = 1;  // this workgroup's share of its unit's key blocks: cut of min(splits, ...)
   // A grid of one workgroup per CU or fewer runs at once in any order and skips
   // the search (15 sequences of 22 to 176 tokens, 16 heads over 2: 18.4 us with
   // it, 16.6 without; nine chunks of 664 rows, 8 heads over 8, 57.9 and 57.5).
-  if (a.n_seqs <= kOrderSeqs && (kCut || gridDim.x > unsigned(kCus))) {
+  // So does a call with a workspace that turns out to cut nothing, as one of
+  // short contexts in a wide table does (the same prompts in tables of 2048
+  // blocks: 19.0 us, of which 1.9 are the combine's launch; 22.3 with the search
+  // and a combine that finds the same out again).
+  if (a.n_seqs <= kOrderSeqs && (kCut || a.n_wg > kCus)) {
     UnitOrder o;
     load_lengths(a, o);
     const EqualPlace e = equal_place(a, int(blockIdx.x));
-    if (!kCut && all_equal(o)) {
+    if constexpr (kCut) {
+      price_cuts(a, o);
+      splits = o.splits;
+      if (blockIdx.x == 0 && threadIdx.x == 0) *a.ws_splits = splits;
+    }
+    if (splits == 1 && all_equal(o)) {
       equal_unit(o, e, u);
       if (u.qb < 0) return;  // uniform
+    } else if (kCut && splits == 1 && a.n_wg <= kCus) {
+      if (int(blockIdx.x) >= a.n_wg) return;  // uniform
+      pair_place(a, u);
+      u.q_begin = __builtin_amdgcn_readlane(o.first, u.b), u.q_len = __builtin_amdgcn_readlane(o.qlen, u.b);
+      u.ctx = __builtin_amdgcn_readlane(o.before, u.b) + u.q_len;
     } else {
-      load_order<kCut>(a, o);
-      splits = o.splits;
+      if (splits == 1) count_units(a, o);
       int r = int(blockIdx.x);
       if (kCut && splits > 1) {  // uniform
         r /= splits;
@@ -405,22 +447,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
       unit_of_rank(a, o, r, u);
     }
   } else {
-    // More sequences, or a small grid: ids are remapped so that all query blocks of one
-    // (sequence, KV head), which stream the same K/V pages, run on one XCD
-    // and share its L2; an XCD holding ppx whole pairs takes query rank
-    // k / ppx of pair k % ppx, its longest causal blocks first.
-    const int n_full = int(gridDim.x) & ~7;
-    const int id = blockIdx.x;
-    const int per_xcd = n_full >> 3;
-    int k = id >> 3;
-    if (per_xcd > 0 && per_xcd % a.n_qb == 0) {
-      const int ppx = per_xcd / a.n_qb;
-      k = (k % ppx) * a.n_qb + k / ppx;
-    }
-    const int unit = id < n_full ? (id & 7) * per_xcd + k : id;
-    const int pair = unit / a.n_qb;
-    u.qb = a.n_qb - 1 - (unit - pair * a.n_qb);
-    u.kvh = pair % a.n_kv_heads, u.b = pair / a.n_kv_heads;
+    pair_place(a, u);
     u.q_begin = a.cu_q[u.b], u.q_len = a.cu_q[u.b + 1] - u.q_begin, u.ctx = a.ctx_lens[u.b];
   }
   // Wave-uniform, and in scalar registers: left to the compiler (their last
@@ -793,13 +820,15 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   uint4 tr[kTu][2];
   if (wave < 4) {
     softmax_phase(kb0, true, -INFINITY);
-    // The place of this loop's code is fixed: it ran 7% slower (one sequence of
-    // 16500 keys: 445 us against 417) in every build that had its first
-    // instruction 4 bytes off a multiple of 8, and any change before it moved
-    // it there.  (s_nop fills the gap, once per workgroup.)
+    // The place of the loops' code is fixed: they ran 7% slower (one sequence
+    // of 16500 keys: 445 us against 417) in a build that had their first
+    // instructions 4 bytes off a multiple of 8, and any change before them moved
+    // them there.  (s_nop fills the gaps, here once per workgroup, in the loops
+    // once a step at most.)
     asm volatile(".p2align 6");
 #pragma nounroll
     for (int kb = kb0; kb < u_end; ++kb) {
+      asm volatile(".p2align 3");
       barrier_after_softmax(true);
       issue_step(kb);
       matrix_phase(kb);
@@ -810,6 +839,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
     }
 #pragma nounroll
     for (int kb = u_end; kb < nkb; ++kb) {
+      asm volatile(".p2align 3");
       barrier_after_softmax(true);
       issue_step(kb);
       matrix_phase(kb);
@@ -822,6 +852,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
     asm volatile(".p2align 6");
 #pragma nounroll
     for (int kb = kb0; kb < u_end; ++kb) {
+      asm volatile(".p2align 3");
       const float ninf = barrier_before_softmax(true);
       issue_step(kb);
       transpose_read(kb + 1, tr);
@@ -832,6 +863,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
     }
 #pragma nounroll
     for (int kb = u_end; kb < nkb; ++kb) {
+      asm volatile(".p2align 3");
       const float ninf = barrier_before_softmax(true);
       issue_step(kb);
       transpose_read(kb + 1, tr);
@@ -872,50 +904,54 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
 }
 
 // Merge the cuts of a unit: M = max m_c, O = sum O_c 2^(m_c - M) / sum l_c
-// 2^(m_c - M) (the rescaling of flash_attn.rs:42-71 across cuts).  grid.x =
-// rank of the unit, grid.y = wave of its workgroup; wave dt of this one
-// takes dims 32 dt .. 32 dt + 31.  Units that are not cut were stored by the
-// main kernel.
+// 2^(m_c - M) (the rescaling of flash_attn.rs:42-71 across cuts).  An item is
+// (rank of the unit, wave of its workgroup); wave dt of this one takes dims
+// 32 dt .. 32 dt + 31.  Units that are not cut were stored by the main kernel;
+// where it cut none, this one reads that and ends.
+constexpr int kCombineWgs = 512;
 template <bool kBf16>
 __global__ __launch_bounds__(64 * (kD / 32)) void paged_prefill_combine(PrefillArgs a, int n_waves) {
+  const int splits = *a.ws_splits;
+  if (splits == 1) return;  // uniform
   UnitOrder ord;
   load_lengths(a, ord);
-  load_order<true>(a, ord);
-  const int r = int(blockIdx.x), wave = int(blockIdx.y);
-  if (ord.splits == 1 || r >= ord.n_units) return;  // uniform
-  PrefillUnit u;
-  unit_of_rank(a, ord, r, u);
-  const int cuts = unit_cuts(ord.splits, key_blocks(unit_keys(a, u.q_len, u.ctx, u.qb)));
-  if (cuts == 1) return;  // uniform
+  count_units(a, ord);
   const int lane = int(threadIdx.x & 63), dt = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int tile = wave / a.group, head = u.kvh * a.group + (wave - tile * a.group);
-  const int qi = (u.qb * a.q_tiles + tile) * kQB + (lane & 31);
-  const int64_t t0 = int64_t(r) * ord.splits * n_waves + wave;  // cut c: t0 + c n_waves
-  const float2* const ml = a.ws_ml + t0 * 64 + lane;
-  const float4* const wo = a.ws_o + (t0 * 16 + 4 * dt) * 64 + lane;
-  float M = -INFINITY;
+  for (int item = int(blockIdx.x); item < ord.n_units * n_waves; item += int(gridDim.x)) {  // uniform
+    const int r = item / n_waves, wave = item - r * n_waves;
+    PrefillUnit u;
+    unit_of_rank(a, ord, r, u);
+    const int cuts = unit_cuts(splits, key_blocks(unit_keys(a, u.q_len, u.ctx, u.qb)));
+    if (cuts == 1) continue;  // uniform
+    const int tile = wave / a.group, head = u.kvh * a.group + (wave - tile * a.group);
+    const int qi = (u.qb * a.q_tiles + tile) * kQB + (lane & 31);
+    const int64_t t0 = int64_t(r) * splits * n_waves + wave;  // cut c: t0 + c n_waves
+    const float2* const ml = a.ws_ml + t0 * 64 + lane;
+    const float4* const wo = a.ws_o + (t0 * 16 + 4 * dt) * 64 + lane;
+    float M = -INFINITY;
 #pragma unroll 4
-  for (int c = 0; c < cuts; ++c) M = fmaxf(M, ml[int64_t(c) * n_waves * 64].x);
-  float acc[4][4] = {}, l = 0.0f;
+    for (int c = 0; c < cuts; ++c) M = fmaxf(M, ml[int64_t(c) * n_waves * 64].x);
+    float acc[4][4] = {}, l = 0.0f;
 #pragma unroll 4
-  for (int c = 0; c < cuts; ++c) {
-    const float2 x = ml[int64_t(c) * n_waves * 64];
-    const float w = x.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(x.x - M);
-    l = fmaf(x.y, w, l);
+    for (int c = 0; c < cuts; ++c) {
+      const float2 x = ml[int64_t(c) * n_waves * 64];
+      const float w = x.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(x.x - M);
+      l = fmaf(x.y, w, l);
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const float4 v = wo[(int64_t(c) * n_waves * 16 + g4) * 64];
-      acc[g4][0] = fmaf(v.x, w, acc[g4][0]);
-      acc[g4][1] = fmaf(v.y, w, acc[g4][1]);
-      acc[g4][2] = fmaf(v.z, w, acc[g4][2]);
-      acc[g4][3] = fmaf(v.w, w, acc[g4][3]);
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const float4 v = wo[(int64_t(c) * n_waves * 16 + g4) * 64];
+        acc[g4][0] = fmaf(v.x, w, acc[g4][0]);
+        acc[g4][1] = fmaf(v.y, w, acc[g4][1]);
+        acc[g4][2] = fmaf(v.z, w, acc[g4][2]);
+        acc[g4][3] = fmaf(v.w, w, acc[g4][3]);
+      }
     }
-  }
-  if (qi >= u.q_len) return;
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  const int64_t orow = ((int64_t(u.q_begin) + qi) * a.n_heads + head) * kD;
+    if (qi >= u.q_len) continue;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const int64_t orow = ((int64_t(u.q_begin) + qi) * a.n_heads + head) * kD;
 #pragma unroll
-  for (int g4 = 0; g4 < 4; ++g4) store4<kBf16>(a, orow + 32 * dt + 8 * g4 + 4 * (lane >> 5), acc[g4], l, inv);
+    for (int g4 = 0; g4 < 4; ++g4) store4<kBf16>(a, orow + 32 * dt + 8 * g4 + 4 * (lane >> 5), acc[g4], l, inv);
+  }
 }
 
 template <bool kBf16, int W, bool kTab, bool kCut>
@@ -948,22 +984,32 @@ hipError_t launch_prefill(const PrefillArgs& a, dim3 grid, hipStream_t s) {
   }
   if (e != hipSuccess || a.max_tiles == 0) return e;
   // Units are cut only where two cuts of all of them fit the workspace.
-  hipLaunchKernelGGL(paged_prefill_combine<kBf16>, dim3(unsigned(a.max_tiles / 2), unsigned(waves)), dim3(64 * (kD / 32)), 0, s,
-                     a, waves);
+  const int items = std::min(a.n_wg, a.max_tiles / 2) * waves;
+  hipLaunchKernelGGL(paged_prefill_combine<kBf16>, dim3(unsigned(std::min(items, kCombineWgs))), dim3(64 * (kD / 32)), 0, s, a,
+                     waves);
   return hipGetLastError();
 }
 
 // Tiles of a workspace that lets a call's units be cut over their keys; 0
-// where they would not be: 512 workgroups or more fill the chip without, and
-// a table of fewer than 32 key blocks a sequence (half a unit's time at 4
-// cuts) gains less than the combine's launch costs.
+// where they would not be: 512 workgroups or more fill the chip without, and a
+// table of fewer than 32 key blocks a sequence (half a unit's time at 4 cuts)
+// gains less than the combine's launch costs.  The units of one sequence are
+// as many as the workgroups; more than 256 have no room for two cuts, and in
+// eight waves the kernel without cuts is the faster (4000 rows of 32 heads over
+// 8: 136.1 us, with a workspace 139.6; not so in seven, whose loops the
+// compiler keeps shorter in the other kernel: 2100 rows, 28 over 4, 68.3 and
+// 67.2).  A unit's cuts hold kCutMin key blocks or more.
 int64_t prefill_tiles(int group, int n_kv_heads, int n_seqs, int max_q_len, int64_t max_keys) {
   const int wg_q = kQB * prefill_q_tiles(group);
   const int64_t n_wg = (int64_t(max_q_len) + wg_q - 1) / wg_q * n_kv_heads * n_seqs;
   if (n_seqs > kOrderSeqs || n_wg == 0 || n_wg >= 512 || max_keys < 32 * kKB) return 0;
-  return std::min<int64_t>(kMaxTiles, n_wg * kMaxCuts);
+  if (n_seqs == 1 && 2 * n_wg > kMaxTiles && group * prefill_q_tiles(group) == 8) return 0;
+  const int64_t cuts = std::min<int64_t>(kMaxCuts, (max_keys + kKB - 1) / kKB / kCutMin);
+  return std::min<int64_t>(kMaxTiles, n_wg * cuts);
 }
 constexpr int64_t kTileWaveBytes = 64 * (16 * 16 + 8);  // a wave's O^T registers and (m, l)
+constexpr int64_t kWsHead = 256;                        // ws_splits
+int64_t prefill_ws_bytes(int64_t tiles, int64_t waves) { return tiles ? kWsHead + tiles * waves * kTileWaveBytes : 0; }
 }  // namespace
 
 extern "C" size_t it_paged_prefill_workspace(int32_t n_heads, int32_t n_kv_heads, int32_t n_seqs, int32_t max_q_len,
@@ -974,7 +1020,7 @@ extern "C" size_t it_paged_prefill_workspace(int32_t n_heads, int32_t n_kv_heads
   const int group = n_heads / n_kv_heads;
   if (group > kMaxGroup) return 0;
   const int64_t tiles = prefill_tiles(group, n_kv_heads, n_seqs, max_q_len, int64_t(max_blocks) * block_size);
-  return size_t(tiles * group * prefill_q_tiles(group) * kTileWaveBytes);
+  return size_t(prefill_ws_bytes(tiles, int64_t(group) * prefill_q_tiles(group)));
 }
 
 extern "C" int32_t it_paged_prefill(const it_kv_cache* c, const void* q, int32_t q_dtype, int32_t n_heads,
@@ -1036,6 +1082,7 @@ extern "C" int32_t it_paged_prefill_ws(const it_kv_cache* c, const void* q, int3
   a.n_seqs = n_seqs;
   const int64_t n_wg = int64_t(a.n_qb) * c->n_kv_heads * n_seqs;
   if (n_wg > INT32_MAX) return fail(IT_INVALID_INPUT, "%s: %lld workgroups (max 2^31 - 1)", who, (long long)n_wg);
+  a.n_wg = int(n_wg);
   const int64_t pairs = int64_t(c->n_kv_heads) * n_seqs, ranks = std::max<int64_t>(n_wg, kMaxTiles);
   a.place = pairs % 8 == 0 ? divisor(pairs / 8, ranks / 8) : divisor(pairs, ranks);
   a.heads = divisor(c->n_kv_heads, pairs);
@@ -1043,11 +1090,11 @@ extern "C" int32_t it_paged_prefill_ws(const it_kv_cache* c, const void* q, int3
   if (ws) {
     if (reinterpret_cast<uintptr_t>(ws) & 255u) return fail(IT_INVALID_INPUT, "%s: ws must be 256-byte aligned", who);
     const int64_t tiles = prefill_tiles(group, c->n_kv_heads, n_seqs, max_q_len, int64_t(max_blocks) << c->log2_bs);
-    const int64_t waves = int64_t(group) * a.q_tiles;
-    if (ws_bytes < size_t(tiles * waves * kTileWaveBytes))
-      return fail(IT_INVALID_INPUT, "%s: workspace %zu < %zu bytes", who, ws_bytes, size_t(tiles * waves * kTileWaveBytes));
+    const int64_t waves = int64_t(group) * a.q_tiles, need = prefill_ws_bytes(tiles, waves);
+    if (ws_bytes < size_t(need)) return fail(IT_INVALID_INPUT, "%s: workspace %zu < %zu bytes", who, ws_bytes, size_t(need));
     a.max_tiles = int(tiles);
-    a.ws_o = static_cast<float4*>(ws);
+    a.ws_splits = static_cast<int*>(ws);
+    a.ws_o = reinterpret_cast<float4*>(static_cast<char*>(ws) + kWsHead);
     a.ws_ml = reinterpret_cast<float2*>(a.ws_o + tiles * waves * 16 * 64);
     if (tiles > n_wg) grid.x = unsigned(tiles);
   }

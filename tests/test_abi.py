@@ -169,6 +169,10 @@ def test_compiled_bindings_agree_with_ctypes():
         assert L.call.it_paged_decode_workspace(*args) == L.lib.it_paged_decode_workspace(*args)
     assert L.call.it_paged_prefill_workspace(32, 8, 1, 500, 1032, 16) == L.lib.it_paged_prefill_workspace(32, 8, 1, 500, 1032, 16) > 0
     assert L.call.it_paged_prefill_workspace(32, 8, 8, 512, 160, 16) == 0  # 512 workgroups without cuts
+    assert L.call.it_paged_prefill_workspace(32, 8, 1, 4000, 250, 16) == 0  # 504 units of one sequence: no room for two cuts
+    assert L.call.it_paged_prefill_workspace(16, 2, 15, 176, 127, 16) == 0 < L.call.it_paged_prefill_workspace(16, 2, 15, 176, 128, 16)
+    tile = 8 * 64 * (16 * 16 + 8)  # 8 waves' partials
+    assert L.call.it_paged_prefill_workspace(32, 8, 1, 64, 128, 16) == 256 + 8 * 4 * tile  # 2048 keys: 4 cuts of 8 units
     ctx, out = np.array([1024, 4096, 17], np.int32), C.c_int32()
     assert L.call.it_paged_decode_partition(L.BF16, 128, 16, 28, 4, ctx, None, 3, 256, out) == L.OK
     want = C.c_int32()

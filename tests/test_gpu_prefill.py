@@ -259,3 +259,49 @@ def test_prefill_units_cut_over_keys(dt, hq, hkv, ctx, q_lens, causal):
                                 260, dctx.data_ptr(), len(ctx), scale, int(causal), plain.data_ptr(), 0,
                                 torch.cuda.current_stream().cuda_stream) == 0
     assert_close(got, from_dev(plain), RTOL, ATOL, what="cut against uncut")
+
+
+@pytest.mark.parametrize("dt,n_seqs,hq,hkv,equal,mb,causal", [
+    (orc.BF16, 5, 16, 2, False, 260, True),    # few workgroups: the order without a search
+    (orc.F16, 5, 7, 1, True, 260, True),       # equal sequences
+    (orc.BF16, 22, 24, 3, False, 260, True),   # 264 workgroups: searched
+    (orc.BF16, 24, 24, 3, True, 260, True),
+    (orc.BF16, 3, 10, 2, False, 13000, False),  # block ids by scalar loads
+])
+def test_prefill_short_contexts_in_wide_tables(dt, n_seqs, hq, hkv, equal, mb, causal):
+    """Tables wide enough that contexts may be long, over contexts that are
+    short: the call takes a workspace and cuts nothing.  With a bound on the
+    contexts it takes none.  Both give the oracle's rows and the same bits, and
+    the bounded call allocates its output alone."""
+    import torch
+    from infer_train_amd import lib
+
+    rng = np.random.RandomState(40 + n_seqs)
+    q_lens = np.full(n_seqs, 97) if equal else rng.choice([0, 1, 31, 33, 65, 100], n_seqs)
+    q_lens[0] = 97
+    ctx = q_lens + (63 if equal else rng.choice([0, 1, 63, 64, 200], n_seqs))
+    dev, ref, tables, ctx, cu, q, td = _setup(dt, hq, hkv, ctx, q_lens, seed=40 + n_seqs, mb=mb)
+    assert lib.it_paged_prefill_workspace(hq, hkv, n_seqs, 97 if equal else int(max(q_lens)), mb, 16) > 0
+    out, scale = _run(dev, tables, ctx, cu, q, td, hq, causal=causal)
+    want = ref.prefill(widen(q, dt), hq, cu, tables, ctx, scale, causal=causal)
+    assert_close(from_dev(out), want, RTOL, ATOL, what=f"wide table n_seqs={n_seqs}")
+    args = to_dev(q.view(np.int16), td), to_dev(cu), int(max(q_lens)), to_dev(tables), to_dev(ctx)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    bounded = dev.prefill(*args, scale=scale, causal=causal, out_dtype=torch.float32, max_ctx_len=int(ctx.max()))
+    assert torch.cuda.max_memory_allocated() - before <= bounded.numel() * 4 + 512
+    np.testing.assert_array_equal(from_dev(bounded), from_dev(out))
+
+
+def test_prefill_bound_of_long_contexts_changes_nothing():
+    """A bound that leaves room for cuts: the call is the one without it."""
+    import torch
+
+    dev, ref, tables, ctx, cu, q, td = _setup(orc.BF16, 16, 2, [2100], [1100], seed=61, mb=260)
+    out, scale = _run(dev, tables, ctx, cu, q, td, 16)  # 70 units of 8 waves, 3 cuts: more merges than the combine has workgroups
+    want = ref.prefill(widen(q, orc.BF16), 16, cu, tables, ctx, scale, causal=True, threads=8)
+    assert_close(from_dev(out), want, RTOL, ATOL, what="cut prefill of 70 units")
+    again = dev.prefill(to_dev(q.view(np.int16), td), to_dev(cu), 1100, to_dev(tables), to_dev(ctx), scale=scale,
+                        out_dtype=torch.float32, max_ctx_len=np.int64(2100))
+    np.testing.assert_array_equal(from_dev(again), from_dev(out))
