@@ -296,7 +296,12 @@ class PagedKvCache:
             held = -(-int(max_ctx_len) // self.block_size)
             if not call.it_paged_prefill_workspace(n_heads, self.n_kv_heads, n_seqs, max_q_len, held, self.block_size):
                 need = 0
-        ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+        ws = None
+        if need:
+            try:
+                ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+            except torch.OutOfMemoryError:
+                need = 0  # the call runs without: only its division over the keys needs memory
         _check(call.it_paged_prefill_ws(self._at, _ptr(q), torch_dtype_id(q.dtype), n_heads, _ptr(cu_q), max_q_len,
                                       _ptr(block_tables), max_blocks, _ptr(ctx_lens), n_seqs, scale,
                                       int(bool(causal)), _ptr(ws), need, _ptr(out), torch_dtype_id(out.dtype),

@@ -305,3 +305,31 @@ def test_prefill_bound_of_long_contexts_changes_nothing():
     again = dev.prefill(to_dev(q.view(np.int16), td), to_dev(cu), 1100, to_dev(tables), to_dev(ctx), scale=scale,
                         out_dtype=torch.float32, max_ctx_len=np.int64(2100))
     np.testing.assert_array_equal(from_dev(again), from_dev(out))
+
+
+def test_prefill_without_memory_for_its_workspace():
+    """A device too full for the workspace: the call runs without one, with
+    the bits of a call that never asked for it."""
+    import torch
+    from infer_train_amd import lib
+
+    dev, ref, tables, ctx, cu, q, td = _setup(orc.BF16, 16, 2, [2100], [1100], seed=62, mb=260)
+    need = lib.it_paged_prefill_workspace(16, 2, 1, 1100, 260, 16)
+    assert need > 32 << 20
+    scale = 0.0884
+    dq, dcu, dtab, dctx = to_dev(q.view(np.int16), td), to_dev(cu), to_dev(tables), to_dev(ctx)
+    out, plain = (torch.empty(q.shape, dtype=torch.float32, device="cuda") for _ in range(2))
+    assert lib.it_paged_prefill(dev.handle, dq.data_ptr(), dev.dtype, 16, dcu.data_ptr(), 1100, dtab.data_ptr(), 260,
+                                dctx.data_ptr(), 1, scale, 1, plain.data_ptr(), 0,
+                                torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(need, dtype=torch.uint8, device="cuda")
+        dev.prefill(dq, dcu, 1100, dtab, dctx, scale=scale, out=out)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    np.testing.assert_array_equal(from_dev(out), from_dev(plain))
