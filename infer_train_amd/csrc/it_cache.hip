@@ -375,10 +375,12 @@ __global__ __launch_bounds__(kThreads) void kv_gather_vec(
 // they are packed in a wave-private LDS stage (wave_lds_fence keeps the
 // order) and stored as 16-byte vectors, or 4- or 2-byte ones where the run
 // starts unaligned (groups of a row that is not a multiple of 8 records).
-// blockIdx.x holds (KV head, 256 groups); blockIdx.y is the sequence.
+// kStage false: each lane stores its record in 2-byte pieces, for small gathers
+// (gather_quant).  blockIdx.x holds (KV head, 256 groups); blockIdx.y is the
+// sequence.
 // Bound by memory: 4 sequences of 4096 to 16384 tokens, 4 x 256, Q8_0 (194
-// MB): 41.0 us, 4.7 TB/s (2-byte stores straight to the records: 46.9 us);
-// small gathers wait for the stage (1.4 MB of 16 sequences: 3.3 us against 2.9).
+// MB): 41.1 us from HBM, 4.7 TB/s, 30 us when the last-level cache holds it
+// (2-byte stores straight to the records: 46.9 us from HBM).
 template <int DT>
 struct GatherRec {
   static constexpr int kBytes = NibFmt<DT>::kRecord;
@@ -388,7 +390,7 @@ struct GatherRec<IT_Q8_0> {
   static constexpr int kBytes = IT_BLOCK_Q8_0_BYTES;
 };
 
-template <int DT>
+template <int DT, bool kStage>
 __global__ __launch_bounds__(kThreads) void kv_gather_quant(
     const char* __restrict__ kpool, const char* __restrict__ vpool, const int32_t* __restrict__ bt,
     int max_blocks, const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ start_pos,
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(kThreads) void kv_gather_quant(
     int64_t num_blocks, unsigned head_wgs, char* __restrict__ kout, char* __restrict__ vout, uint32_t* err) {
   constexpr int REC = GatherRec<DT>::kBytes;
   constexpr bool kQ8 = DT == IT_Q8_0;
-  __shared__ __attribute__((aligned(16))) char stage[kThreads / 64][2][64 * REC];
+  __shared__ __attribute__((aligned(16))) char stage[kStage ? kThreads / 64 : 1][2][kStage ? 64 * REC : 16];
   const int b = blockIdx.y;
   const int st = start_pos ? start_pos[b] : 0;
   const int n = ctx_lens[b] - st;
@@ -455,10 +457,11 @@ __global__ __launch_bounds__(kThreads) void kv_gather_quant(
   const int n_rec = int(min(int64_t(64), total - wave0));
   const int64_t rec0 = ((cu_out[b] * hkv + int64_t(h) * n) * ng + wave0) * REC;
   const bool whole = __builtin_amdgcn_ballot_w64(live && !found) == 0;  // no record of the wave is skipped
+  if (!kStage && !(live && found)) return;
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
-    char* const sg = stage[threadIdx.x >> 6][w];
-    uint16_t* o = reinterpret_cast<uint16_t*>(sg + lane * REC);
+    char* const to = kStage ? stage[threadIdx.x >> 6][w] : (w ? vout : kout) + rec0;
+    uint16_t* o = reinterpret_cast<uint16_t*>(to + lane * REC);
     auto put = [&](uint32_t x) {
       o[0] = uint16_t(x & 0xFFFFu);
       o[1] = uint16_t(x >> 16);
@@ -479,6 +482,7 @@ __global__ __launch_bounds__(kThreads) void kv_gather_quant(
       put(q[w][c].w);
     }
   }
+  if constexpr (!kStage) return;
   wave_lds_fence();
   const char* const sk = stage[threadIdx.x >> 6][0];
   const char* const sv = stage[threadIdx.x >> 6][1];
@@ -524,6 +528,17 @@ __global__ __launch_bounds__(kThreads) void kv_gather_quant(
   } else {
     copy(uint16_t{});
   }
+}
+
+// Workgroups (of the grid; lengths may leave some without work) from which
+// records go through the stage: below, the wait for it shows, above, the
+// 2-byte stores do.  us staged / direct (4 x 256 and 8 x 128 alike), 128
+// workgroups: Q8_0 3.28 / 3.22, Q4_0 2.89 / 2.80, Q5_0 3.16 / 2.91; 256: Q8_0
+// 3.69 / 3.87, Q4_0 3.06 / 2.96, Q5_0 3.39 / 3.30, Q4_1 and Q5_1 equal; 512:
+// Q8_0 4.71 / 5.44, Q4_0 3.62 / 3.60, Q5_0 4.17 / 4.28, Q4_1 3.50 / 3.74.
+template <int DT>
+auto* gather_quant(int64_t wgs) {
+  return wgs >= (DT == IT_Q4_0 || DT == IT_Q5_0 ? 512 : 256) ? kv_gather_quant<DT, true> : kv_gather_quant<DT, false>;
 }
 
 // ---------------------------------------------------------------------------
@@ -877,11 +892,12 @@ extern "C" int32_t it_kv_gather(const it_kv_cache* c, const int32_t* bt, int32_t
   if (is_quant(c->dtype)) {
     const int64_t head_wgs = cdiv(int64_t(max_tokens) * (c->head_dim / 32), kThreads);
     dim3 grid(unsigned(head_wgs * c->n_kv_heads), unsigned(n_seqs));
-    auto* kern = c->dtype == IT_Q8_0   ? kv_gather_quant<IT_Q8_0>
-                 : c->dtype == IT_Q4_0 ? kv_gather_quant<IT_Q4_0>
-                 : c->dtype == IT_Q4_1 ? kv_gather_quant<IT_Q4_1>
-                 : c->dtype == IT_Q5_0 ? kv_gather_quant<IT_Q5_0>
-                                       : kv_gather_quant<IT_Q5_1>;
+    const int64_t wgs = int64_t(grid.x) * n_seqs;
+    auto* kern = c->dtype == IT_Q8_0   ? gather_quant<IT_Q8_0>(wgs)
+                 : c->dtype == IT_Q4_0 ? gather_quant<IT_Q4_0>(wgs)
+                 : c->dtype == IT_Q4_1 ? gather_quant<IT_Q4_1>(wgs)
+                 : c->dtype == IT_Q5_0 ? gather_quant<IT_Q5_0>(wgs)
+                                       : gather_quant<IT_Q5_1>(wgs);
     hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, s,
                        (const char*)c->k_pool, (const char*)c->v_pool,
                        bt, max_blocks, ctx_lens, start_pos, cu_out, c->n_kv_heads, c->head_dim, c->log2_bs,

@@ -476,8 +476,9 @@ def test_append_nibble_chunks_and_scales(dt, D, hkv, n):
 @pytest.mark.parametrize("dt", [orc.Q8_0, orc.Q4_0, orc.Q4_1, orc.Q5_0, orc.Q5_1])
 @pytest.mark.parametrize("D,shift", [(32, 0), (32, 2), (96, 4), (128, 8), (256, 6)])
 def test_gather_records_at_any_alignment(dt, D, shift):
-    """Packed records through the 64-record stage: rows of 1, 3, 4 and 8
-    groups, runs that start on 2-, 4- and 16-byte boundaries, sequences that
+    """Packed records through the 64-record stage (a bound on the tokens of 512
+    workgroups) and straight from the lanes (the small gather's own bound): rows
+    of 1, 3, 4 and 8 groups, runs that start on 2-, 4- and 16-byte boundaries, sequences that
     end inside a wave; nothing around them is written.  A block id outside the
     pool is latched and leaves exactly its records as they were."""
     import torch
@@ -498,7 +499,7 @@ def test_gather_records_at_any_alignment(dt, D, shift):
     cu = np.concatenate([[0], np.cumsum(n)[:-1]]).astype(np.int64)
     rk, rv = ref.gather(tables, ctx, start, cu, int(n.sum()))
     row = D // 32 * orc.RECORD_BYTES[dt]
-    for bad in (False, True):
+    for bad, max_tokens in ((bad, m) for bad in (False, True) for m in (int(n.max()), 43 * 256 * 32 // D)):
         t = tables.copy()
         hole = np.zeros(rk.size, bool)
         if bad:
@@ -507,7 +508,7 @@ def test_gather_records_at_any_alignment(dt, D, shift):
                 at = (int(cu[2]) * hkv + h * int(n[2]) + 80 - 7) * row
                 hole[at:at + 16 * row] = True
         bufs = [torch.full((rk.size + 64,), 0xEE, dtype=torch.uint8, device="cuda:0") for _ in range(2)]
-        dev.gather(to_dev(t), to_dev(ctx), to_dev(start), to_dev(cu), int(n.max()), *(x[shift:] for x in bufs))
+        dev.gather(to_dev(t), to_dev(ctx), to_dev(start), to_dev(cu), max_tokens, *(x[shift:] for x in bufs))
         if bad:
             with pytest.raises(InvalidInput):
                 dev.check()
