@@ -356,6 +356,10 @@ size_t it_paged_decode_workspace(int32_t n_seqs, int32_t n_heads, int32_t head_d
  * units beyond the resident slots would run a second round.  A batch that
  * needs more than two rounds at any size takes the longest partition that
  * keeps two workgroups per compute unit instead (fewest partials).
+ * Quantised caches at head_dim 128 run up to eight workgroups per unit (six
+ * for some head counts): where four would take partitions above 384 tokens, the
+ * same is planned over the partitions that leave room for all of them (or
+ * seven), and the longest is that which leaves room for all.
  *   ctx_lens, start_pos: host int32[n_seqs] (start_pos may be NULL)
  *   n_cu: compute units of the device (0 = ask the current HIP device)
  * No counterpart in the reference: flash_attn_f32 (flash_attn.rs:6-72) does

@@ -172,11 +172,11 @@ extern "C" int32_t it_paged_decode_partition(int32_t dtype, int32_t head_dim, in
     const int64_t n = int64_t(ctx_lens[b]) - (start_pos ? start_pos[b] : 0);
     if (n > max_n) max_n = n;
   }
-  // Resident slots of one round: `cap` workgroups of two waves per compute
-  // unit (half of four-wave ones past four), fewer where the LDS does not
-  // hold them.
+  // Resident slots of one round: four workgroups per compute unit, fewer where
+  // the LDS does not hold four.  `full`: as many two-wave ones as the registers
+  // hold, of the partitions that leave the LDS room for all of them (or seven).
   struct Plan {
-    int best = 0, longest = 0;  // fewest rounds; longest that keeps the unit full (two workgroups, past cap 4 every one)
+    int best = 0, longest = 0;  // fewest rounds; longest that keeps two workgroups (full: all) per unit
     int64_t rounds = 0;
   };
   auto plan = [&](bool full) {
@@ -187,8 +187,14 @@ extern "C" int32_t it_paged_decode_partition(int32_t dtype, int32_t head_dim, in
       const SplitShape sh = split_shape(dtype, head_dim, gc, p, (p >> log2_bs) + 2, parts * hc * n_seqs);
       const size_t smem = split_lds_bytes(dtype, head_dim, gc, p, (p >> log2_bs) + 2, sh.nw, sh.ring);
       if (smem > kMaxDecodeLds) continue;
-      const int cap = full ? split_resident(dtype, head_dim, sh.nw) : 4;
-      const int64_t per_cu = std::min<int64_t>(cap, int64_t(kMaxDecodeLds / smem));
+      int cap = 2;
+      int64_t per_cu = std::min<int64_t>(4, int64_t(kMaxDecodeLds / smem));
+      if (full) {
+        if (sh.nw != 2) continue;  // four-wave ones: 6% slower (Q5_1, 11 sequences of 55530 tokens, 6 heads over one)
+        cap = split_resident(dtype, head_dim, gc);
+        per_cu = std::min<int64_t>(cap, int64_t(kMaxDecodeLds / ((smem + kLdsPiece - 1) / kLdsPiece * kLdsPiece)));
+        if (per_cu < std::min(cap, 7)) continue;
+      }
       int64_t units = 0;
       for (int b = 0; b < n_seqs; ++b) {
         const int64_t n = int64_t(ctx_lens[b]) - (start_pos ? start_pos[b] : 0);
@@ -199,23 +205,31 @@ extern "C" int32_t it_paged_decode_partition(int32_t dtype, int32_t head_dim, in
         r.best = p;
         r.rounds = rounds;
       }
-      if (per_cu >= (full ? cap : 2)) r.longest = p;
+      if (per_cu >= cap) r.longest = p;
     }
     return r;
   };
   Plan r = plan(false);
-  // Where registers hold more workgroups, long partitions run shorter beside
-  // more of them.  Short ones stay: 320 tokens at four per unit 28.3 us, 192
-  // at eight 29.3 (32 sequences of 256 to 4096 tokens, 7 heads over one).
-  if (split_resident(dtype, head_dim, 2) > 4 && r.best > 384) {
+  // Where registers hold more workgroups, long partitions give way to the
+  // shorter ones that leave room for them: over 700 batches (1 to 64 sequences
+  // of up to 65536 tokens, windows, ten head counts, five block sizes, the five
+  // formats) 0.88 of the time at four per unit on average, 1.03 or less for 98%
+  // of them.  With partitions of four to six among them, or counted as eight
+  // where registers or LDS hold fewer, up to 1.5 (Q4_0, 9 sequences of 53787
+  // tokens, 32 heads over 8: 2048 tokens at three workgroups of four waves 193
+  // us, 1984 at four of two waves 280, 768 at eight 169).  Partitions of 384
+  // tokens and fewer stay: from 256 on, 1.06 for 5% of the batches, and twice the
+  // partials of one long sequence cost its merge more (Q4_0, 45656 tokens, 64
+  // heads over 8: 384 tokens 31.9 us, 192 35.1).
+  if (split_resident(dtype, head_dim, gc) > 4 && r.best > 384) {
     const Plan f = plan(true);
-    if (f.best && (f.rounds <= 2 || f.longest)) r = f;
+    if (f.best) r = f;
   }
   if (!r.best) return fail(IT_NOT_IMPLEMENTED, "%s: no partition fits (max context %lld)", who, (long long)max_n);
   // Beyond two rounds the workgroups stream back to back and the machine
-  // stays full whatever the size: then the longest partition that still
-  // keeps the compute units full (two workgroups each; see above) writes the
-  // fewest partials and starts the fewest workgroups.
+  // stays full whatever the size: then the longest partition (of two workgroups
+  // per unit or more; see above) writes the fewest partials and starts the
+  // fewest workgroups.
   *partition = (r.rounds > 2 && r.longest) ? r.longest : r.best;
   return IT_OK;
 }

@@ -167,15 +167,29 @@ inline SplitShape split_shape(int32_t dt, int d, int gc, int partition, int max_
   return {4, 2};
 }
 
-// Workgroups of a launch shape that run on one CU, as far as registers go
-// (LDS may hold fewer).  The quantised formats at head_dim 128 take 113-116
-// VGPRs: four waves per SIMD.  Their items are short (16 tokens: 64 bytes a
-// row) and each is a chain of waits, conversions and MFMAs, so four waves
-// hide what two do not; more ring slots did not (Q4_0, 16 sequences of 2048 to
-// 16384 tokens, 8 KV heads: 640-token partitions, eight workgroups per CU,
-// 65 us; 1344 tokens, four, 97 us; three or four slots 67-100 us).  The other
-// kernels: four workgroups (more were slower for the 16-bit formats).
-inline int split_resident(int32_t dt, int d, int nw) { return is_quant(dt) && d == 128 ? 16 / nw : 4; }
+// Waves per SIMD that the registers of the two-wave kernels hold (1: four
+// workgroups per CU are planned whatever they hold; more were slower for the
+// 16-bit formats).  The quantised formats at head_dim 128 run four: their items
+// are short (16 tokens: 64 bytes a row) and each is a chain of waits,
+// conversions and MFMAs, so four waves hide what two do not; more ring slots did
+// not (Q4_0, 16 sequences of 2048 to 16384 tokens, 8 KV heads: 640-token
+// partitions, eight workgroups per CU, 65 us; 1344 tokens, four, 97 us; three or
+// four slots 67-100 us).  The kernel's launch bounds hold it to their 128 VGPRs:
+// left alone the compiler took 130 to 133 for Q5_1 and two of Q4_1's head
+// counts, which is three waves, and a plan of four ran a second round (Q4_1, 32
+// sequences of 4096, 7 heads over one: 55.9 us; held 43.5; four workgroups per
+// CU 47.2).  Four of Q5_1's head counts would spill for it (4% slower) and run
+// three.
+constexpr int split_waves(int dt, int d, int gc) {
+  const bool quant = dt == IT_Q8_0 || dt == IT_Q4_0 || dt == IT_Q4_1 || dt == IT_Q5_0 || dt == IT_Q5_1;
+  return !quant || d != 128 ? 1 : dt == IT_Q5_1 && (gc == 2 || (gc >= 5 && gc <= 7)) ? 3 : 4;
+}
+// Workgroups of two waves that run on one CU as far as registers go, as planned for.
+inline int split_resident(int32_t dt, int d, int gc) { return is_quant(dt) && d == 128 ? 2 * split_waves(dt, d, gc) : 4; }
+// LDS is given out in pieces of 1280 bytes: 32284 bytes are four to a CU, not
+// five (Q4_0, 8 sequences of 32768 tokens, 7 heads over one: 832-token
+// partitions at five per CU 98 us, 1024 at four 64 us).
+constexpr size_t kLdsPiece = 1280;
 
 // Compile-time loop: f(integral_constant<int, I>) for I in [B, E).
 template <int B, int E>
@@ -455,7 +469,7 @@ __device__ __forceinline__ void fold8(const float (&x)[8], float& ra, float& rb)
 }
 
 template <int DT, int D, int GC, int NW, int R>
-__global__ __launch_bounds__(64 * NW) void paged_decode_split(DecodeArgs a) {
+__global__ __launch_bounds__(64 * NW, (NW == 2 ? split_waves(DT, D, GC) : 1)) void paged_decode_split(DecodeArgs a) {
   using F = SplitFmt<DT, D>;
   constexpr int RB = F::kRow, GB = F::kGroup, SLOT = F::kSlot, NI = F::kDma, NL = F::kLoads;
   constexpr int PQ = F::kPieces, NQ = F::kQRegs, DPV = F::kDpv;

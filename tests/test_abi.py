@@ -153,6 +153,12 @@ def test_decode_partition_planner_quantised_128():
     assert plan(even, 32, 8, L.BF16) != 576
     # 32 x 1024 over 4 KV heads: 128-token partitions at four per unit, kept.
     assert plan(np.full(32, 1024), 28, 4, L.Q4_0) == 128
+    # Only partitions that leave room for eight (LDS is given out in pieces of 1280 bytes): not 832 tokens at
+    # four of what looks like five, nor the 1984 that run in the fewest rounds of four.
+    assert plan(np.full(8, 32768), 28, 4, L.Q4_0) == 256
+    assert plan(np.full(9, 53787), 32, 8, L.Q4_0) == 832
+    # Registers for three waves (Q5_1, 7 heads): six workgroups per unit, not eight.
+    assert plan(np.full(32, 4096), 28, 4, L.Q5_1) > plan(np.full(32, 4096), 28, 4, L.Q5_0) == 256
     # Many rounds at any size: the longest partition that leaves room for eight.
     long = plan(np.full(16, 65536), 32, 8, L.Q4_0)
     assert 640 <= long <= 1024

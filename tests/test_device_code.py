@@ -80,3 +80,46 @@ def test_wave_private_lds_stages_are_fenced(tmp_path):
     assert all(n in names for n in ("kv_append_q8_wide", "kv_append_nib_wide", "kv_gather_quant"))
     bad = {k: b for k, b in ((k, _unordered(v)) for k, v in staged.items()) if b}
     assert not bad, {k: b[:3] for k, b in bad.items()}
+
+
+def _kernel_registers():
+    """{kernel: (VGPRs, spilled VGPRs)} of the built library's code objects."""
+    import struct
+
+    from infer_train_amd._lib import LIB_PATH
+
+    readelf = "/opt/rocm/llvm/bin/llvm-readelf"
+    if not os.path.exists(readelf):
+        pytest.skip("llvm-readelf not found")
+    data = open(LIB_PATH, "rb").read()
+    magic, found, at = b"__CLANG_OFFLOAD_BUNDLE__", {}, 0
+    while (at := data.find(magic, at)) >= 0:
+        p = at + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", data, p - 8)[0]):
+            off, size, n = struct.unpack_from("<QQQ", data, p)
+            if b"gfx950" in data[p + 24:p + 24 + n] and size:
+                notes = subprocess.run([readelf, "--notes", "-"], input=data[at + off:at + off + size], capture_output=True,
+                                       check=True).stdout.decode()
+                for block in notes.split(".agpr_count:")[1:]:
+                    name, v, s = (re.search(rf"\.{key}:\s+(\S+)", block) for key in ("name", "vgpr_count", "vgpr_spill_count"))
+                    found[name[1]] = int(v[1]), int(s[1])
+            p += 24 + n
+        at += len(magic)
+    return found
+
+
+def test_decode_registers_allow_the_planned_waves():
+    """The partition planner counts on the waves that a SIMD's 512 VGPRs hold
+    (allocated in eights) of the quantised decode at head_dim 128 in two-wave
+    workgroups: four, three for four of Q5_1's head counts; none of them spills."""
+    from infer_train_amd import _lib as L
+
+    regs, seen = _kernel_registers(), 0
+    for name, (vgprs, spilled) in regs.items():
+        m = re.search(r"paged_decode_splitILi(\d+)ELi128ELi(\d+)ELi2ELi2E", name)
+        if not m or int(m[1]) not in (L.Q4_0, L.Q4_1, L.Q5_0, L.Q5_1, L.Q8_0):
+            continue
+        seen += 1
+        want = 3 if int(m[1]) == L.Q5_1 and int(m[2]) in (2, 5, 6, 7) else 4
+        assert 512 // (-(-vgprs // 8) * 8) >= want and spilled == 0, (name, vgprs, spilled)
+    assert seen == 5 * 8  # formats, head counts
