@@ -148,25 +148,23 @@ __global__ __launch_bounds__(kThreads) void kv_append_rope(RopeAppendArgs a) {
 }
 
 // The same for rows of a power of two of 16-byte vectors, four up to a wave
-// (head_dim 16, 32, 64, 128 or 256; other widths take the kernel above).  A wave takes one token: its position, slot
-// and angles (one 16-byte load per lane) are read once and serve kRowGroups
-// instructions of RPI = 64 / vecs (token, head) rows each, q's, k's and v's
-// heads numbered one after another; all rows are loaded before the first is
-// stored.  Bound by memory: 4096 tokens of 32 + 2 x 8 heads of 128, bf16
-// cache (151 MB): 28.8 us, 5.2 TB/s, a large copy's rate (one vector per lane,
-// its (token, head) found by 64-bit divisions, in a grid of three parts each
-// sized for q: 47.3 us).  Two rows a lane 30.6, eight 30.9; without the
-// non-temporal hint on the loads 30.8.
-constexpr int kRowGroups = 4;
-
-template <int DT>
+// (head_dim 16, 32, 64, 128 or 256; other widths take the kernel above).  A wave
+// takes one token: its position, slot and angles are read once and serve G
+// instructions of RPI = 64 / vecs (token, head) rows each, q's, k's and v's heads
+// numbered one after another; all rows are loaded before the first is stored.
+// Bound by memory: 4096 tokens of 32 + 2 x 8 heads of 128, bf16 cache (151 MB):
+// 28.8 us, 5.2 TB/s, a large copy's rate (one vector per lane, its (token, head)
+// found by 64-bit divisions, in a grid of three parts each sized for q: 47.3 us).
+// Two rows a lane 30.6, eight 30.9; without the non-temporal hint on the loads
+// 30.8.  Small calls are a chain of waits, longer with each row: see launch_rope.
+template <int DT, int G>
 __global__ __launch_bounds__(kThreads) void kv_append_rope_rows(RopeAppendArgs a, int log2_vecs) {
   const int64_t t = int64_t(blockIdx.x) * (kThreads / 64) + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   if (t >= a.n_tokens) return;  // uniform
   const int lane = int(threadIdx.x & 63), vecs = 1 << log2_vecs, cv = lane & (vecs - 1);
   const int rpi = 64 >> log2_vecs;
   const int rows = a.hq + 2 * a.hkv;
-  const int row0 = int(blockIdx.y) * (rpi * kRowGroups) + (lane >> log2_vecs);
+  const int row0 = int(blockIdx.y) * (rpi * G) + (lane >> log2_vecs);
   const int pos = a.positions[t];
   const int64_t slot = a.slots[t];
   // A token whose position is outside the table writes nothing (K, V or q).
@@ -174,9 +172,9 @@ __global__ __launch_bounds__(kThreads) void kv_append_rope_rows(RopeAppendArgs a
     if (blockIdx.y == 0 && lane == 0) atomicOr(a.err, kErrPos);
     return;
   }
-  float4 x[kRowGroups];
+  float4 x[G];
 #pragma unroll
-  for (int j = 0; j < kRowGroups; ++j) {
+  for (int j = 0; j < G; ++j) {
     // Past the last row a lane re-reads it; only the stores are predicated.
     const int r = min(row0 + j * rpi, rows - 1);
     const int rk = r - a.hq, rv = rk - a.hkv;
@@ -196,7 +194,7 @@ __global__ __launch_bounds__(kThreads) void kv_append_rope_rows(RopeAppendArgs a
   const int64_t off = slot & ((int64_t(1) << a.log2_bs) - 1);
   const bool cached = slot >= 0 && slot < a.n_slots;  // uniform
 #pragma unroll
-  for (int j = 0; j < kRowGroups; ++j) {
+  for (int j = 0; j < G; ++j) {
     const int r = row0 + j * rpi;
     const int rk = r - a.hq, rv = rk - a.hkv;
     if (r >= rows) continue;
@@ -220,17 +218,28 @@ __global__ __launch_bounds__(kThreads) void kv_append_rope_rows(RopeAppendArgs a
   }
 }
 
+template <int DT, int G>
+void launch_rows(const RopeAppendArgs& a, int vecs, int64_t chunks, hipStream_t s) {
+  const dim3 grid(unsigned((a.n_tokens + kThreads / 64 - 1) / (kThreads / 64)), unsigned(chunks));
+  hipLaunchKernelGGL((kv_append_rope_rows<DT, G>), grid, dim3(kThreads), 0, s, a, ilog2(vecs));
+}
+
+// Rows per lane: one, two or four, the fewest with which all waves are resident
+// at once (32 of 256 CUs).  us with one / two / four, bf16: one token of 32 + 2 x
+// 8 heads of 128 2.23 / 2.61 / 3.31 (a vector per lane: 2.49), 128 tokens 2.79 /
+// 3.11 / 3.98, 256 3.62 / 3.52 / 4.17, 512 5.54 / 4.93 / 5.19, 1024 9.34 / 8.51 /
+// 7.97; Q8_0, 128 tokens 3.20 / 3.89 / 4.86, 1024 11.1 / 10.7 / 11.1.
+constexpr int64_t kRopeWaves = 256 * 32;
+
 template <int DT>
 void launch_rope(const RopeAppendArgs& a, hipStream_t s) {
   const int vecs = a.d / 4;
   if (vecs >= 4 && vecs <= 64 && (vecs & (vecs - 1)) == 0) {
-    const int per = 64 / vecs * kRowGroups;  // rows per wave
-    const int64_t chunks = (int64_t(a.hq) + 2 * int64_t(a.hkv) + per - 1) / per;
-    if (chunks <= 65535) {
-      const dim3 grid(unsigned((a.n_tokens + kThreads / 64 - 1) / (kThreads / 64)), unsigned(chunks));
-      hipLaunchKernelGGL(kv_append_rope_rows<DT>, grid, dim3(kThreads), 0, s, a, ilog2(vecs));
-      return;
-    }
+    const int64_t rows = int64_t(a.hq) + 2 * int64_t(a.hkv);
+    const auto chunks = [&](int g) { return (rows + 64 / vecs * g - 1) / (64 / vecs * g); };  // waves per token
+    if (chunks(1) <= 65535 && a.n_tokens * chunks(1) <= kRopeWaves) return launch_rows<DT, 1>(a, vecs, chunks(1), s);
+    if (chunks(2) <= 65535 && a.n_tokens * chunks(2) <= kRopeWaves) return launch_rows<DT, 2>(a, vecs, chunks(2), s);
+    if (chunks(4) <= 65535) return launch_rows<DT, 4>(a, vecs, chunks(4), s);
   }
   const int64_t blocks = (a.n_tokens * a.hq * vecs + kThreads - 1) / kThreads;  // Q has the most rows
   hipLaunchKernelGGL(kv_append_rope<DT>, dim3(unsigned(blocks), 3), dim3(kThreads), 0, s, a);

@@ -417,13 +417,16 @@ def test_append_rope_bad_position_is_latched():
     (orc.Q4_0, 32, 7, 7, 4, 32),     # 8 rows an instruction
     (orc.F32, 16, 2, 1, 6, 4),       # the narrowest row taken so: 16 rows an instruction
     (orc.BF16, 96, 4, 2, 5, 96),     # not a power of two: one vector per lane
+    # 24 rows of 128: 8192 waves at 682 tokens of one row a lane and 1365 of two
+    (orc.BF16, 128, 16, 4, 682, 128), (orc.Q5_1, 128, 16, 4, 683, 128),
+    (orc.Q8_0, 128, 16, 4, 1365, 128), (orc.F32, 128, 16, 4, 1366, 128),
 ])
 def test_append_rope_row_shapes(dt, D, hq, hkv, n, n_dims):
     """Head counts that do not fill a wave's rows, every row width, partly
     rotated rows: pools and rotated q equal the oracle's byte for byte."""
     from infer_train_amd.kv import RopeTable
 
-    nb, bs = 8, 16
+    nb, bs = max(8, -(-n // 16)), 16
     dev, ref = _pair(nb, bs, hkv, D, dt)
     rope = RopeTable(n_dims, 300)
     rng = np.random.default_rng(D)
