@@ -102,10 +102,12 @@ __device__ __forceinline__ bool q8_fast_scale(float scale) { return scale >= 0x1
 // at most `top`.  r = x id + half + 0.5 with |x| <= |max| and id = 1 / (max /
 // -half), or (x - min) id + 0.5 with id = 1 / ((max - min) / top): when id is
 // finite d is at least 2^-128, rounded by 2^-22 at most, so r lies in (0, 2
-// half + 1); else the product is infinite or NaN.  So r is a small positive
-// number or the code is 0, and an unsigned convert and one bound say which.
-__device__ __forceinline__ uint32_t quant_code(float r, uint32_t top) {
-  return min(uint32_t(r < 64.0f ? r : 0.0f), top);  // NaN fails the compare; r > -1
+// half + 1); else the product is infinite (of either sign) or NaN.  So r is a
+// small positive number or the code is 0, and an unsigned convert and one bound
+// say which.
+__host__ __device__ __forceinline__ uint32_t quant_code(float r, uint32_t top) {
+  const uint32_t c = uint32_t(__builtin_fabsf(r) < 64.0f ? r : 0.0f);  // NaN and the infinities fail the compare
+  return c < top ? c : top;
 }
 
 // Steps of a reduction over an 8-lane group in which the lower lane wins

@@ -123,3 +123,37 @@ def test_decode_registers_allow_the_planned_waves():
         want = 3 if int(m[1]) == L.Q5_1 and int(m[2]) in (2, 5, 6, 7) else 4
         assert 512 // (-(-vgprs // 8) * 8) >= want and spilled == 0, (name, vgprs, spilled)
     assert seen == 5 * 8  # formats, head counts
+
+
+_QUANT_CODE = r"""
+#include <cmath>
+#include <cstdio>
+#include "it_device.hpp"
+#include "it_quant.hpp"
+using namespace itkv;
+int main() {
+  const float inf = INFINITY, r[] = {0.0f, -0.0f, 0.49f, 0.999f, 1.0f, 8.5f, 15.99f, 16.0f, 31.5f, 32.99f, inf, -inf, NAN, -NAN};
+  const unsigned want[] = {0, 0, 0, 0, 1, 8, 15, 16, 31, 32, 0, 0, 0, 0};
+  for (unsigned top : {15u, 31u})
+    for (int i = 0; i < 14; ++i) {
+      const unsigned w = want[i] < top ? want[i] : top;
+      if (quant_code(r[i], top) != w) return printf("%g: %u, not %u\n", double(r[i]), quant_code(r[i], top), w), 1;
+    }
+  return 0;
+}
+"""
+
+
+def test_quant_code_is_defined_for_every_value(tmp_path):
+    """quant_code on the host, with conversions out of range trapped: the
+    infinities of an overflowed 1 / d have the code 0 of a NaN."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not found")
+    src, exe = tmp_path / "code.hip", str(tmp_path / "code")
+    src.write_text(_QUANT_CODE)
+    cmd = [HIPCC, "--offload-arch=gfx950", "-std=c++17", "-O1", "-I", CSRC, "-I", os.path.join(ROOT, "include"),
+           "-Xarch_host", "-fsanitize=float-cast-overflow", "-Xarch_host", "-fsanitize-trap=all", str(src), "-o", exe]
+    b = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
+    assert b.returncode == 0, b.stderr[-2000:]
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stdout)
