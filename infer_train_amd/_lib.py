@@ -183,7 +183,7 @@ def _load_call():
     try:
         from . import _call
     except ImportError as e:
-        raise ImportError(f"{_HERE}/_call.so is missing or does not load ({e}): build it with "
+        raise ImportError(f"{_HERE}/_call (this interpreter's binding) is missing or does not load ({e}): build it with "
                           "`python -c 'import __graft_entry__ as g; g.build()'`") from e
     _call.bind(LIB_PATH, lib)
     return _call

@@ -257,3 +257,21 @@ def test_compiled_bindings_take_and_refuse_what_ctypes_does():
         out.value = 0
         assert L.call.it_paged_decode_partition(*planner[:5], ctx.ctypes.data, None, n, 256, C.addressof(out)) == L.OK
         assert out.value > 0
+
+
+def test_compiled_bindings_belong_to_this_interpreter(monkeypatch):
+    """The binding is built with the headers of the interpreter that runs
+    build(), under its ABI's name, so that another one does not load it."""
+    import subprocess
+    import sys
+    import sysconfig
+
+    import __graft_entry__ as entry
+    from infer_train_amd import _lib as L
+
+    assert L.call.__file__.endswith("_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+    calls = []
+    monkeypatch.setattr(subprocess, "run", lambda cmd, **kw: calls.append(cmd))
+    entry.build()
+    csrc = [c for c in calls if any(x.endswith("csrc") for x in c)]
+    assert len(csrc) == 1 and f"PYTHON={sys.executable}" in csrc[0]
