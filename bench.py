@@ -1017,7 +1017,7 @@ def movers_plan():
          q8_tok * 4 * d256 * 4 * 2, q8_tok * 4 * d256 * 34 // 32 * 2),
         ("gather_bf16_c2_4k", "kv_gather_vec", "gather of config 2 at 4k: 32 x 4096 tokens, bf16, Hkv 4",
          g_tok * 4 * d128 * bf * 2, g_tok * 4 * d128 * bf * 2),
-        ("gather_q8_0_c5", "kv_gather_q8_0", "gather of 4 x 8192 Q8_0 tokens as BlockQ8_0 records, Hkv 4, D 256",
+        ("gather_q8_0_c5", "kv_gather_quant<8", "gather of 4 x 8192 Q8_0 tokens as BlockQ8_0 records, Hkv 4, D 256",
          gq_tok * 4 * d256 * 34 // 32 * 2, gq_tok * 4 * d256 * 34 // 32 * 2),
         ("clear_blocks_4096", "kv_clear_blocks", "evict 4096 config-4 blocks (2 heads x 4 KiB, K and V)",
          ev_big * 4, ev_big * 2 * 4096 * 2),
@@ -1176,6 +1176,8 @@ def summarize_movers_profile(d, args):
             ids = sorted(i for kn, s in by_kernel.items() if ksub in kn for i in s)
             start = used.get(ksub, 0)
             mine = ids[start:start + MOVER_WARM + MOVER_REPS]
+            if rs and len(mine) < MOVER_WARM + MOVER_REPS:
+                raise SystemExit(f"{name}: {len(mine)} launches of a kernel named {ksub}, not {MOVER_WARM + MOVER_REPS}")
             used[ksub] = start + MOVER_WARM + MOVER_REPS
             out[name] = set(mine[MOVER_WARM:])
         return out
@@ -1560,9 +1562,9 @@ def summarize_config5_profile(d, args):
 ISA_KERNELS = [
     ("it_decode_bf16.hip", "paged_decode_splitILi30ELi128ELi7ELi2ELi2E", "split-K decode, bf16, D 128, 7 heads, 2 waves, 2-slot rings (config 2 headline)"),
     ("it_decode_q8_0.hip", "paged_decode_splitILi8ELi256ELi6ELi4ELi2E", "split-K decode, Q8_0, D 256, 6 heads, 4 waves (config 5)"),
-    ("it_attn.hip", "paged_decode_combineILi128E", "combine pass, D 128"),
-    ("it_prefill.hip", "paged_prefill_kernelILb1ELi8ELb1E", "chunked prefill, bf16, 8 waves (config 3)"),
-    ("it_cache.hip", "kv_append_copy", "append, bit copy"),
+    ("it_attn.hip", "paged_decode_combineILi128ELi1E", "combine pass, D 128, one wave a row"),
+    ("it_prefill.hip", "paged_prefill_kernelILb1ELi8ELb1ELb0E", "chunked prefill, bf16, 8 waves (config 3)"),
+    ("it_cache.hip", "kv_append_copyE", "append, bit copy"),
     ("it_cache.hip", "kv_append_quantILi8E", "quantise-append, Q8_0"),
     ("it_cache.hip", "kv_gather_vec", "block-table gather, 16/32-bit caches"),
     ("it_cache.hip", "kv_clear_blocks", "evict (page clear)"),
@@ -1615,8 +1617,7 @@ def isa_census(args):
         text = asm[src]
         m = re.search(r"^(_Z\S*" + sym + r"\S*):", text, re.M)
         if not m:
-            rows.append((src, sym, what, None, None))
-            continue
+            raise SystemExit(f"{src}: no kernel named {sym}")
         name = m.group(1)
         body = text[m.end():text.index(".Lfunc_end", m.end())]
         counts = {c: 0 for c, _ in ISA_CLASSES}
@@ -1647,9 +1648,6 @@ def isa_census(args):
     lines.append("| " + " | ".join(hdr) + " |")
     lines.append("|" + "---|" * len(hdr))
     for src, sym, what, counts, meta in rows:
-        if counts is None:
-            lines.append(f"| `{sym}` | {what} | not found |")
-            continue
         vals = [str(counts[c]) for c, _ in ISA_CLASSES]
         mv = [str(meta.get(k, "")) for k in ("vgpr_count", "agpr_count", "sgpr_count", "vgpr_spill_count")]
         lines.append(f"| `{sym}` ({src}) | {what} | " + " | ".join(vals + mv) + " |")

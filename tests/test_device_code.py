@@ -157,3 +157,17 @@ def test_quant_code_is_defined_for_every_value(tmp_path):
     assert b.returncode == 0, b.stderr[-2000:]
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout)
+
+
+def test_profiled_kernels_exist():
+    """The kernels that the profile summaries look for are in the library: the
+    movers' by name, the instruction census's exactly one each."""
+    import bench
+
+    names = list(_kernel_registers())
+    for workload, kernel, *_ in bench.movers_plan():
+        base, _, arg = kernel.partition("<")
+        symbol = base + (f"ILi{arg}E" if arg else "")
+        assert any(symbol in n for n in names), workload
+    for _, symbol, _ in bench.ISA_KERNELS:
+        assert sum(symbol in n for n in names) == 1, symbol
