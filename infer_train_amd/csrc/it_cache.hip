@@ -316,9 +316,11 @@ __global__ __launch_bounds__(kThreads) void kv_append_nib_wide(
 }
 
 // Fewest chunks it is used for.  A wave quantises its eight instructions one
-// after another, which costs appends that leave SIMDs idle 1.2 to 2 us (Q4_0 /
-// Q5_1): 256 chunks 4.4 us so against 3.5 a vector per lane, 512 4.6 / 5.8
-// against 4.7 / 5.3, 1024 5.9 (Q4_0) against 7.9.
+// after another, which costs appends that leave SIMDs idle 1.2 to 2 us.  us wide /
+// a vector per lane, 4 x 256: 256 chunks Q4_0 4.04 / 3.26, Q5_1 5.23 / 3.69; 512
+// Q4_0 4.23 / 4.27, Q4_1 5.15 / 4.76, Q5_0 4.66 / 4.61, Q5_1 5.49 / 5.02; 768 5.10
+// / 5.30, 6.12 / 5.92, 5.53 / 5.73, 6.64 / 6.29; 1024 5.39 / 6.38, 6.47 / 7.14,
+// 5.82 / 6.90, 6.82 / 7.59; 8 x 64 at 1024 6.65 / 7.20 (Q4_0), 8.55 / 8.45 (Q5_1).
 constexpr int64_t kWideChunks = 768;
 
 template <int DT>

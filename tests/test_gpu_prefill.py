@@ -230,25 +230,59 @@ def test_prefill_unit_order_past_one_round(n_seqs, hq, hkv, equal, causal):
     assert_close(from_dev(out), want, RTOL, ATOL, what=f"prefill order n_seqs={n_seqs} equal={equal}")
 
 
-@pytest.mark.parametrize("dt,hq,hkv,ctx,q_lens,causal", [
-    (orc.BF16, 8, 2, [2100], [70], True),          # one long context, few rows: 8 cuts
-    (orc.F16, 7, 1, [4096, 130], [33, 1], True),   # 7 waves; a unit too short to cut beside long ones
-    (orc.BF16, 5, 1, [2049, 0, 3000], [1, 0, 129], True),  # 5 waves, an empty sequence, the diagonal inside the last cut
-    (orc.BF16, 2, 2, [2111], [300], False),        # 8 query tiles a workgroup, every key visible
-    (orc.BF16, 8, 1, [1100, 1023], [64, 64], True),  # at the edge: 17 and 16 key blocks
+def _expected_cuts(hq, hkv, ctx, q_lens, causal, tiles):
+    """The number of cuts the device prices from a call's lengths (blocks of 64
+    keys, a cut costs five, at least eight a cut, 256 workgroups at once)."""
+    group = hq // hkv
+    rows = 32 * (1 if group >= 8 else 8 // group)
+    blocks = lambda keys: max((keys + 63) // 64, 0)  # noqa: E731
+    units = work = most = 0
+    for c, q in zip(ctx, q_lens):
+        n = -(-q // rows)
+        if n == 0:
+            continue
+        first, last = (blocks(c - q + (min(q, x) if causal else q)) for x in (rows, n * rows))
+        units += n * hkv
+        work += n * (first + last) // 2
+        most = max(most, last)
+    if most < 16 or units == 0 or 2 * units > tiles:
+        return 1
+    mean, best = hkv * work * 16 // units, None
+    for cuts in range(1, 17):
+        if cuts > 1 and (units * cuts > tiles or most < 8 * cuts):
+            break
+        extra = 80 if cuts > 1 else 0
+        cost = max(-(-units * cuts // 256) * (mean // cuts + extra), 16 * most // cuts + extra)
+        cost -= cost // 10 if cuts == 1 else 0
+        if best is None or cost < best[0]:
+            best = cost, cuts
+    return best[1]
+
+
+@pytest.mark.parametrize("dt,hq,hkv,ctx,q_lens,causal,mb,cuts", [
+    (orc.BF16, 8, 2, [2100], [70], True, 260, 4),          # one long context, few rows: 33 key blocks
+    (orc.F16, 7, 1, [4096, 130], [33, 1], True, 260, 8),   # 7 waves; a unit too short to cut beside long ones
+    (orc.BF16, 5, 1, [2049, 0, 3000], [1, 0, 129], True, 260, 5),  # 5 waves, an empty sequence, the diagonal inside the last cut
+    (orc.BF16, 2, 2, [2111], [300], False, 260, 4),        # 8 query tiles a workgroup, every key visible
+    (orc.BF16, 8, 1, [1100, 1023], [64, 64], True, 260, 2),  # at the edge: 18 and 16 key blocks
+    (orc.BF16, 8, 2, [2100, 1500], [70, 40], True, 13000, 4),  # a table too wide for LDS: block ids by scalar loads
+    (orc.F16, 6, 2, [5000], [33], False, 7200, 9),
 ])
-def test_prefill_units_cut_over_keys(dt, hq, hkv, ctx, q_lens, causal):
+def test_prefill_units_cut_over_keys(dt, hq, hkv, ctx, q_lens, causal, mb, cuts):
     """Launches of few units divide each unit's key blocks among several
     workgroups and merge their partial (m, l, O).  Against the oracle, and
     against the same call without a workspace (no cuts): the two differ by
-    the rounding of the 16-bit probabilities to different maxima."""
+    the rounding of the 16-bit probabilities to different maxima.  The number of
+    cuts the device took is the one priced here."""
     import torch
     from infer_train_amd import lib
 
     gain = lambda p: 1.0 + (p % 700) / 300.0  # noqa: E731  cuts with different maxima
-    dev, ref, tables, ctx, cu, q, td = _setup(dt, hq, hkv, ctx, q_lens, seed=900 + hq, mb=260, k_gain=gain)
-    need = lib.it_paged_prefill_workspace(hq, hkv, len(ctx), int(max(q_lens)), 260, 16)
-    assert need > 0
+    raw_ctx, raw_q = list(ctx), list(q_lens)
+    dev, ref, tables, ctx, cu, q, td = _setup(dt, hq, hkv, ctx, q_lens, seed=900 + hq, mb=mb, k_gain=gain)
+    need = lib.it_paged_prefill_workspace(hq, hkv, len(ctx), int(max(q_lens)), mb, 16)
+    waves = hq // hkv * (1 if hq // hkv >= 8 else 8 // (hq // hkv))
+    assert _expected_cuts(hq, hkv, raw_ctx, raw_q, causal, (need - 256) // (waves * 64 * 264)) == cuts
     out, scale = _run(dev, tables, ctx, cu, q, td, hq, causal=causal)
     want = ref.prefill(widen(q, dt), hq, cu, tables, ctx, scale, causal=causal)
     got = from_dev(out)
@@ -256,9 +290,15 @@ def test_prefill_units_cut_over_keys(dt, hq, hkv, ctx, q_lens, causal):
     dq, plain = to_dev(q.view(np.int16), td), torch.empty(q.shape, dtype=torch.float32, device="cuda")
     dcu, dt_, dctx = to_dev(cu), to_dev(tables), to_dev(ctx)
     assert lib.it_paged_prefill(dev.handle, dq.data_ptr(), dev.dtype, hq, dcu.data_ptr(), int(max(q_lens)), dt_.data_ptr(),
-                                260, dctx.data_ptr(), len(ctx), scale, int(causal), plain.data_ptr(), 0,
+                                mb, dctx.data_ptr(), len(ctx), scale, int(causal), plain.data_ptr(), 0,
                                 torch.cuda.current_stream().cuda_stream) == 0
     assert_close(got, from_dev(plain), RTOL, ATOL, what="cut against uncut")
+    ws, own = torch.empty(need, dtype=torch.uint8, device="cuda"), torch.empty_like(plain)
+    assert lib.it_paged_prefill_ws(dev.handle, dq.data_ptr(), dev.dtype, hq, dcu.data_ptr(), int(max(q_lens)), dt_.data_ptr(),
+                                   mb, dctx.data_ptr(), len(ctx), scale, int(causal), ws.data_ptr(), need, own.data_ptr(), 0,
+                                   torch.cuda.current_stream().cuda_stream) == 0
+    np.testing.assert_array_equal(from_dev(own), got)
+    assert int(ws[:4].view(torch.int32).item()) == cuts  # the main kernel leaves the number there for the merge
 
 
 @pytest.mark.parametrize("dt,n_seqs,hq,hkv,equal,mb,causal", [
