@@ -357,8 +357,8 @@ __device__ __forceinline__ void unit_of_rank(const PrefillArgs& a, const UnitOrd
 // blocks of one (sequence, KV head), which stream the same K/V pages, run on
 // one XCD and share its L2; an XCD holding ppx whole pairs takes query rank
 // k / ppx of pair k % ppx, its longest causal blocks first.
-__device__ __forceinline__ void pair_place(const PrefillArgs& a, PrefillUnit& u) {
-  const int n_full = a.n_wg & ~7;
+__device__ __forceinline__ void pair_place(const PrefillArgs& a, int n_wg, PrefillUnit& u) {
+  const int n_full = n_wg & ~7;
   const int id = blockIdx.x;
   const int per_xcd = n_full >> 3;
   int k = id >> 3;
@@ -406,10 +406,6 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   // first ends.  Up to kOrderSeqs sequences: id = rank in the longest-first
   // order (unit_of_rank), so every XCD gets the same share of long and short
   // units whatever the sequences' lengths.
-  // The arguments that place the workgroup, loaded at once (the compiler loads
-  // each where it is used: a round trip after another).
-  asm volatile("" ::"s"(a.cu_q), "s"(a.ctx_lens), "s"(a.n_seqs), "s"(a.n_kv_heads), "s"(a.q_tiles), "s"(a.n_qb), "s"(a.n_wg),
-               "s"(a.causal), "s"(a.group), "s"(a.place.d), "s"(a.place.inv), "s"(a.heads.d), "s"(a.heads.inv));
   PrefillUnit u;
   int cut = 0, splits = 1;  // this workgroup's share of its unit's key blocks: cut of min(splits, ...)
   // A grid of one workgroup per CU or fewer runs at once in any order and skips
@@ -419,7 +415,14 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
   // short contexts in a wide table does (the same prompts in tables of 2048
   // blocks: 19.0 us, of which 1.9 are the combine's launch; 22.3 with the search
   // and a combine that finds the same out again).
-  if (a.n_seqs <= kOrderSeqs && (kCut || a.n_wg > kCus)) {
+  const int n_wg = kCut ? a.n_wg : int(gridDim.x);
+  if (a.n_seqs <= kOrderSeqs && (kCut || n_wg > kCus)) {
+    // The arguments that place the workgroup, loaded at once: the compiler loads
+    // each where it is used, a round trip after another (six ragged prompts 61.2
+    // us so, 60.8 at once).  Not in the small grids below, which need fewer of
+    // them (nine chunks of 16 rows, 6 waves: 17.9 us with it, 17.2 without).
+    asm volatile("" ::"s"(a.cu_q), "s"(a.ctx_lens), "s"(a.n_seqs), "s"(a.n_kv_heads), "s"(a.q_tiles), "s"(a.n_qb), "s"(a.n_wg),
+                 "s"(a.causal), "s"(a.group), "s"(a.place.d), "s"(a.place.inv), "s"(a.heads.d), "s"(a.heads.inv));
     UnitOrder o;
     load_lengths(a, o);
     const EqualPlace e = equal_place(a, int(blockIdx.x));
@@ -431,9 +434,9 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
     if (splits == 1 && all_equal(o)) {
       equal_unit(o, e, u);
       if (u.qb < 0) return;  // uniform
-    } else if (kCut && splits == 1 && a.n_wg <= kCus) {
-      if (int(blockIdx.x) >= a.n_wg) return;  // uniform
-      pair_place(a, u);
+    } else if (kCut && splits == 1 && n_wg <= kCus) {
+      if (int(blockIdx.x) >= n_wg) return;  // uniform
+      pair_place(a, n_wg, u);
       u.q_begin = __builtin_amdgcn_readlane(o.first, u.b), u.q_len = __builtin_amdgcn_readlane(o.qlen, u.b);
       u.ctx = __builtin_amdgcn_readlane(o.before, u.b) + u.q_len;
     } else {
@@ -447,7 +450,7 @@ __global__ __launch_bounds__(64 * W) void paged_prefill_kernel(PrefillArgs a) {
       unit_of_rank(a, o, r, u);
     }
   } else {
-    pair_place(a, u);
+    pair_place(a, n_wg, u);
     u.q_begin = a.cu_q[u.b], u.q_len = a.cu_q[u.b + 1] - u.q_begin, u.ctx = a.ctx_lens[u.b];
   }
   // Wave-uniform, and in scalar registers: left to the compiler (their last
